@@ -58,10 +58,7 @@ struct gs_batch {
     int persistent_groups = 0;
     uint32_t capacity = 0;
     bool direct = true;            // direct-placement binning (else the word sort)
-    int bin_G = 0, bin_C = 0;      // Gaussians per group, groups per view
-    size_t bin_L = 0;              // (view, tile, group) table entries + 1
-    int bin_blocks = 0, bin_tpl = 1;
-    int bin_diff_len = 0;  // largest view's (tiles per row + 1) * (tile rows + 1)
+    gsb::BinArgs bin{};            // direct placement: layout, views and workspace
     int num_cus = 0;
 
     hipStream_t stream = nullptr;
@@ -74,11 +71,11 @@ struct gs_batch {
     DevBuf means2D, depths, conics, op2d, rgb, radii, tiles;
     DevBuf dkeys, didx, dkeys_s, didx_s, rtiles, roff, scan_partial, dsort_ws;
     DevBuf words, words_tmp, tsort_ws, ranges;
-    DevBuf values, bviews_dev, bvblock_dev, bin_table, bin_scanned, bin_partial, bin_rects;
+    DevBuf values, bviews_dev, bin_ws, coarse;
     DevBuf rect_idx;  // direct binning: packed tile rectangles by (view, Gaussian), from the preprocess
     DevBuf image, d_image, gt, T_final, n_contrib, last;
     DevBuf rg;  // screen-space gradients, one block of V*N: means2D (8 B), conics (12), rgb (12), opacities (4)
-    DevBuf losses, l1_partial, small;  // small: total32 @0, total64 @8, overflow @16, skipped @20
+    DevBuf losses, l1_partial, small;  // small: total32 @0, total64 @8, overflow @16, skipped @20, records @24
     int l1_nb = 0;
 
     gs_preprocessed pre() {
@@ -92,6 +89,8 @@ struct gs_batch {
     uint32_t* total32() { return reinterpret_cast<uint32_t*>(small.p); }
     unsigned long long* total64() { return reinterpret_cast<unsigned long long*>(static_cast<char*>(small.p) + 8); }
     uint32_t* overflow() { return reinterpret_cast<uint32_t*>(static_cast<char*>(small.p) + 16); }
+    // bin records of the last binning
+    unsigned long long* records() { return reinterpret_cast<unsigned long long*>(static_cast<char*>(small.p) + 24); }
     // steps whose update the overflow flag suppressed since the last check
     uint32_t* skipped() { return reinterpret_cast<uint32_t*>(static_cast<char*>(small.p) + 20); }
     ~gs_batch();
@@ -102,8 +101,7 @@ gs_batch::~gs_batch() {
     graph.release();
     DevBuf* all[] = {&cams_dev, &views_dev, &pixoff_dev, &hp_dev, &counters, &means2D, &depths, &conics, &op2d, &rgb,
                      &radii, &tiles, &dkeys, &didx, &dkeys_s, &didx_s, &rtiles, &roff, &scan_partial, &dsort_ws,
-                     &words, &words_tmp, &tsort_ws, &ranges, &values, &bviews_dev, &bvblock_dev, &bin_table, &bin_scanned,
-                     &bin_partial, &bin_rects, &image, &d_image, &gt, &T_final, &n_contrib, &last,
+                     &words, &words_tmp, &tsort_ws, &ranges, &values, &bviews_dev, &bin_ws, &coarse, &rect_idx, &image, &d_image, &gt, &T_final, &n_contrib, &last,
                      &rg, &losses, &l1_partial, &small};
     for (DevBuf* b : all) b->release();
     if (ev_in) (void)hipEventDestroy(ev_in);
@@ -144,41 +142,61 @@ static int batch_size_pairs(gs_batch* b, uint32_t cap) {
     return GS_OK;
 }
 
-// Direct-placement binning layout for the current group size / bin shape:
-// groups per view, the (view, tile, group) table and each view's first block.
-static int batch_setup_binning(gs_batch* b, int group, int tpl) {
-    b->bin_G = group;
-    b->bin_tpl = tpl;
-    b->bin_C = (b->N + b->bin_G - 1) / b->bin_G;
-    b->bin_L = (size_t)b->bin_C * (size_t)b->total_tiles + 1;
-    if (b->bin_L >= 0xFFFFFFFFull) return gs_set_error(GS_ERR_INVALID, "binning table too large");
-    const int V = b->V;
-    std::vector<int4> bviews(V);
-    std::vector<int> vblock0(V + 1, 0);
-    size_t tab = 0;
-    b->bin_diff_len = 0;
-    for (int v = 0; v < V; v++) {
-        const int gx = b->views[v].z, gy = (b->views[v].y + 15) / 16;
-        bviews[v] = int4{gx, gy, (int)(uint32_t)tab, b->views[v].w};
-        tab += (size_t)gx * gy * b->bin_C;
-        vblock0[v + 1] = vblock0[v] + bin_blocks(b->bin_C, gx, gy, b->bin_tpl);
-        b->bin_diff_len = std::max(b->bin_diff_len, (gx + 1) * (gy + 1));
-    }
-    b->bin_blocks = vblock0[V];
-    const size_t VN = (size_t)V * b->N;
-    B_TRY(b->bviews_dev.ensure(sizeof(int4) * V));
-    B_TRY(b->bvblock_dev.ensure(sizeof(int) * (V + 1)));
-    B_TRY(b->bin_table.ensure(b->bin_L * 4));
-    B_TRY(b->bin_scanned.ensure(b->bin_L * 4));
-    B_TRY(b->bin_rects.ensure(VN * 8));
-    B_TRY(b->bin_partial.ensure(((b->bin_L + SCAN_BLOCK - 1) / SCAN_BLOCK + 1) * 8));
-    B_HIP(hipMemcpyAsync(b->bviews_dev.p, bviews.data(), sizeof(int4) * V, hipMemcpyHostToDevice, b->stream),
-          "hipMemcpyAsync(views)");
-    B_HIP(hipMemcpyAsync(b->bvblock_dev.p, vblock0.data(), sizeof(int) * (V + 1), hipMemcpyHostToDevice, b->stream),
-          "hipMemcpyAsync(blocks)");
-    B_HIP(hipStreamSynchronize(b->stream), "hipStreamSynchronize");  // the host vectors die here
+// Room for `records` bin records.
+static int batch_size_records(gs_batch* b, size_t records) {
+    records = std::min<size_t>(records, 0xFFFFFFFFu);
+    const size_t bytes = records * bin_record_bytes(b->bin);
+    if (bytes <= b->coarse.bytes) return GS_OK;
     b->graph.release();
     b->graph_ready = false;
+    return b->coarse.ensure(bytes);
+}
+
+static uint32_t batch_record_cap(gs_batch* b) {
+    return (uint32_t)std::min<size_t>(b->coarse.bytes / bin_record_bytes(b->bin), 0xFFFFFFFFu);
+}
+
+// Direct-placement binning layout: the views' first bins and tiles, chunks,
+// groups and workspace.
+static int batch_setup_binning(gs_batch* b) {
+    const int V = b->V;
+    gsb::BinArgs& a = b->bin;
+    a = gsb::BinArgs{};
+    a.V = V;
+    a.N = b->N;
+    a.total_tiles = b->total_tiles;
+    int max_gx = 0, max_gy = 0;
+    for (int v = 0; v < V; v++) {
+        max_gx = std::max(max_gx, b->views[v].z);
+        max_gy = std::max(max_gy, (b->views[v].y + 15) / 16);
+    }
+    a.side = bin_side(max_gx, max_gy);
+    std::vector<int4> bviews(V);
+    for (int v = 0; v < V; v++) {
+        const int gx = b->views[v].z, gy = (b->views[v].y + 15) / 16;
+        const int bins = bin_count_of_view(a.side, gx, gy);
+        bviews[v] = int4{gx, gy, (int)a.NB, b->views[v].w};
+        a.NB += (uint32_t)bins;
+        a.max_bins = std::max(a.max_bins, bins);
+    }
+    B_TRY(b->bviews_dev.ensure(sizeof(int4) * V));
+    B_HIP(hipMemcpyAsync(b->bviews_dev.p, bviews.data(), sizeof(int4) * V, hipMemcpyHostToDevice, b->stream),
+          "hipMemcpyAsync(views)");
+    B_HIP(hipStreamSynchronize(b->stream), "hipStreamSynchronize");  // the host vector dies here
+    a.views = static_cast<const int4*>(b->bviews_dev.p);
+    if (b->N > 0) {
+        bin_layout(a);
+        if (a.table2_len >= 0xFFFFFFFFull || a.table1_len >= 0xFFFFFFFFull)
+            return gs_set_error(GS_ERR_INVALID, "binning table too large");
+        B_TRY(b->bin_ws.ensure(bin_workspace_bytes(a)));
+        bin_carve(a, b->bin_ws.p);
+        // a first guess (2 to 6 records per Gaussian and view are usual); batch_measure grows it
+        B_TRY(batch_size_records(b, 4 * (size_t)V * b->N + 65536));
+    }
+    a.sidx = b->didx_s.u();
+    a.sidx_stride = 1;
+    a.rect_idx = b->rect_idx.u();
+    a.overflow = b->overflow();
     return GS_OK;
 }
 
@@ -254,7 +272,7 @@ extern "C" int gs_batch_create(gs_trainer* tr, int n_views, const gs_camera* cam
     b->l1_nb = std::max(1, std::min(512, (max_pix * 3 + 255) / 256 / 4));
     if ((st = b->l1_partial.ensure((size_t)n_views * b->l1_nb * 8))) return fail(st);
     if (b->direct) {
-        if ((st = batch_setup_binning(b, tr->ctx->bin_chunk, tr->ctx->bin_tpl))) return fail(st);
+        if ((st = batch_setup_binning(b))) return fail(st);
     } else if ((st = b->rtiles.ensure(VN * 4)) || (st = b->roff.ensure(VN * 4))) {
         return fail(st);
     }
@@ -300,7 +318,8 @@ extern "C" int gs_batch_set_targets(gs_batch* b, const float* const* gts, int fr
 }
 
 // Everything from preprocess to the tile ranges (the forward's binning).
-static int enqueue_binning(gs_batch* b, hipStream_t s) {
+// place: false stops at the pair and record counts (batch_measure).
+static int enqueue_binning(gs_batch* b, hipStream_t s, bool place = true) {
     gs_trainer* t = b->tr;
     const uint32_t VN = (uint32_t)((size_t)b->V * b->N);
     gs_gaussians g = t->gaussians();
@@ -315,35 +334,21 @@ static int enqueue_binning(gs_batch* b, hipStream_t s) {
                                  b->radix_bits, b->dsort_ws.p, s, nullptr),
           "depth sort");
     if (b->direct) {
-        gsb::BinArgs a{};
-        a.V = b->V;
-        a.N = b->N;
-        a.C = b->bin_C;
-        a.G = b->bin_G;
-        a.S = 0;
-        a.G1 = b->bin_G;
-        a.sidx = b->didx_s.u();
-        a.sidx_stride = 1;
-        a.means2D = reinterpret_cast<const float2*>(pre.means2D);
-        a.radii = pre.radii;
-        a.views = static_cast<const int4*>(b->bviews_dev.p);
-        a.vblock0 = b->bvblock_dev.i();
-        a.table = b->bin_table.u();
-        a.table_len = b->bin_L;
-        a.rects = static_cast<uint2*>(b->bin_rects.p);
+        gsb::BinArgs a = b->bin;
+        a.coarse = b->coarse.p;
+        a.coarse_cap = batch_record_cap(b);
         a.out = b->values.u();
         a.capacity = b->capacity;
-        a.overflow = b->overflow();
-        a.diff_len = b->bin_diff_len;
-        a.rect_idx = b->rect_idx.u();
-        B_HIP(launch_bin_count(a, b->bin_blocks, b->bin_tpl, s), "binning count");
-        B_HIP(launch_scan_u32_exclusive(b->bin_table.u(), (uint32_t)b->bin_L, b->bin_scanned.u(),
-                                        static_cast<unsigned long long*>(b->bin_partial.p), s, b->total32(),
-                                        b->total64()),
-              "binning scan");
-        a.table = b->bin_scanned.u();
-        B_HIP(launch_bin_place(a, b->bin_blocks, b->bin_tpl, s), "binning place");
-        B_HIP(launch_bin_ranges(a, b->bin_scanned.u(), (uint32_t)b->total_tiles, b->ranges.u(), s), "binning ranges");
+        if (b->N == 0) {  // no lists: every range is empty
+            B_HIP(launch_zero(b->ranges.p, (size_t)b->total_tiles * 8, s), "zero ranges");
+            B_HIP(launch_zero(b->total32(), 16, s), "zero counts");
+            return GS_OK;
+        }
+        B_HIP(launch_bin_lists(a, s, b->records(), b->total32(), b->total64()), "binning lists");
+        if (place) {
+            B_HIP(launch_bin_place(a, s), "binning place");
+            B_HIP(launch_bin_ranges(a, b->ranges.u(), s), "binning ranges");
+        }
         return GS_OK;
     }
     B_HIP(launch_gather_tiles_multi(VN, b->N, static_cast<const uint64_t*>(b->dkeys_s.p), b->didx_s.u(), pre.tiles_touched,
@@ -470,22 +475,35 @@ static int enqueue_step(gs_batch* b, hipStream_t s) {
     return GS_OK;
 }
 
-// Sizes the pair buffers with one binning pass (eager, synchronous).
+// Sizes the pair buffers from a binning pass (eager, synchronous): first the
+// record buffer, whose overflow cuts the pair count short, then the pairs.
+// The overflow flag is cleared when a buffer grew.
 static int batch_measure(gs_batch* b, long long* pairs) {
     if (b->capacity == 0) B_TRY(batch_size_pairs(b, 1024));
-    B_TRY(enqueue_binning(b, b->stream));
-    unsigned long long K = 0;
-    B_HIP(hipMemcpyAsync(&K, b->total64(), 8, hipMemcpyDeviceToHost, b->stream), "hipMemcpyAsync");
-    B_HIP(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
-    if (K > 0xFFFFFFFFull) return gs_set_error(GS_ERR_CAPACITY, "more than 2^32-1 pairs");
-    *pairs = (long long)K;
-    if (K > b->capacity) {
-        unsigned long long cap = K + K / 4 + 65536;
-        if (cap > 0xFFFFFFFFull) cap = 0xFFFFFFFFull;
-        B_TRY(batch_size_pairs(b, (uint32_t)cap));
-        B_HIP(launch_zero(b->overflow(), 4, b->stream), "zero overflow");
+    for (int attempt = 0; attempt < 2; attempt++) {
+        B_TRY(enqueue_binning(b, b->stream, false));
+        unsigned long long K = 0, records = 0;
+        B_HIP(hipMemcpyAsync(&K, b->total64(), 8, hipMemcpyDeviceToHost, b->stream), "hipMemcpyAsync");
+        B_HIP(hipMemcpyAsync(&records, b->records(), 8, hipMemcpyDeviceToHost, b->stream), "hipMemcpyAsync");
+        B_HIP(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
+        if (b->direct && records > batch_record_cap(b)) {
+            if (records > 0xFFFFFFFFull) return gs_set_error(GS_ERR_CAPACITY, "more than 2^32-1 bin records");
+            B_TRY(batch_size_records(b, records + records / 4 + 65536));
+            B_HIP(launch_zero(b->overflow(), 4, b->stream), "zero overflow");
+            continue;
+        }
+        if (K > 0xFFFFFFFFull) return gs_set_error(GS_ERR_CAPACITY, "more than 2^32-1 pairs");
+        *pairs = (long long)K;
+        // the words path places (and drops) pairs while it is measured
+        if (K > b->capacity) {
+            unsigned long long cap = K + K / 4 + 65536;
+            if (cap > 0xFFFFFFFFull) cap = 0xFFFFFFFFull;
+            B_TRY(batch_size_pairs(b, (uint32_t)cap));
+            B_HIP(launch_zero(b->overflow(), 4, b->stream), "zero overflow");
+        }
+        return GS_OK;
     }
-    return GS_OK;
+    return gs_set_error(GS_ERR_CAPACITY, "the bin record buffer did not grow");
 }
 
 static int batch_upload_hparams(gs_batch* b, const gs_train_cfg* tc, int iteration) {
@@ -531,6 +549,13 @@ static int batch_result(gs_batch* b, gs_step_result* out, int iteration) {
         B_HIP(launch_zero(b->overflow(), 8, b->stream), "zero overflow");
         b->tr->adam_steps -= (int)skipped;
         const uint32_t old_cap = b->capacity;
+        if (b->direct) {
+            // records that did not fit cut the pair count short: count again, growing both buffers
+            long long pairs = 0;
+            B_TRY(batch_measure(b, &pairs));
+            K = (unsigned long long)pairs;
+            if (out) out->pairs = pairs;
+        }
         unsigned long long cap = K + K / 4 + 65536;
         if (cap > 0xFFFFFFFFull) cap = 0xFFFFFFFFull;
         B_TRY(batch_size_pairs(b, (uint32_t)cap));
@@ -718,16 +743,10 @@ extern "C" int gs_batch_autotune(gs_batch* b, int reps, gs_tuning* out) {
     res.radix_bits = b->radix_bits;
     res.split_groups = c->split_groups;  // a single-view knob, reported unchanged
     auto bin = [&]() { return enqueue_binning(b, b->stream); };
-    if (b->direct) {
-        B_TRY(batch_pick(b, tm, reps, {1, 2, 4}, [&](int x) { return batch_setup_binning(b, b->bin_G, x); }, bin,
-                         &res.bin_tiles_per_lane, &res.binning_ms));
-        B_TRY(batch_pick(b, tm, reps, {2048, 4096, 8192, 16384, 32768, 65536},
-                         [&](int x) { return batch_setup_binning(b, x, b->bin_tpl); }, bin, &res.bin_group,
-                         &res.binning_ms));
-    } else {
-        int unused = 0;
-        B_TRY(batch_pick(b, tm, reps, {0}, [](int) { return GS_OK; }, bin, &unused, &res.binning_ms));
-    }
+    res.bin_tiles_per_lane = c->bin_tpl;  // knobs without effect, reported unchanged
+    res.bin_group = c->bin_chunk;
+    int unused = 0;
+    B_TRY(batch_pick(b, tm, reps, {0}, [](int) { return GS_OK; }, bin, &unused, &res.binning_ms));
     B_TRY(bin());
     // persistent groups per CU, on forward + loss + backward raster
     const int persistent0 = b->persistent;

@@ -198,7 +198,7 @@ gs_trainer::~gs_trainer() {
 
 void gs::ViewBufs::release_all() {
     DevBuf* all[] = {&means2D, &depths, &conics, &op2d, &rgb, &radii, &tiles, &offsets, &ranges, &image, &d_image,
-                     &T_final, &n_contrib, &last, &loss, &rg, &split_flags, &split_rc};
+                     &T_final, &n_contrib, &last, &loss, &rg};
     for (DevBuf* b : all) b->release();
 }
 
@@ -277,19 +277,25 @@ extern "C" void* gs_trainer_buffer(gs_trainer* t, const char* which) {
 static int tr_bin(gs_trainer* t, gs::ViewBufs& v, const gs_camera* cam, const gs_preprocessed& pre, long long* K) {
     gs_ctx* c = t->ctx;
     const bool words = (cam->width + 15) / 16 > GS_BIN_MAX_TILES_XY || (cam->height + 15) / 16 > GS_BIN_MAX_TILES_XY;
-    const size_t per = words ? 8 : 4;
+    if (!words) {
+        TR_TRY(gs_bin_prepare(c, t->n, &pre, cam->width, cam->height, K, nullptr, nullptr));
+        if ((size_t)*K > t->keys_sorted.bytes / 4) TR_TRY(t->keys_sorted.ensure((size_t)(*K + *K / 8 + 1024) * 4));
+        const uint32_t cap = (uint32_t)std::min<size_t>(t->keys_sorted.bytes / 4, 0xFFFFFFFFu);
+        if (*K > (long long)cap) return gs_set_error(GS_ERR_CAPACITY, "trainer binning: %lld pairs", *K);
+        TR_TRY(gs_bin_finish(c, t->keys_sorted.u(), cap, v.ranges.u()));
+        t->pair_stride = 1;
+        return GS_OK;
+    }
     for (int attempt = 0; attempt < 2; attempt++) {
-        const uint32_t cap = (uint32_t)std::min<size_t>(t->keys_sorted.bytes / per, 0xFFFFFFFFu);
-        int st = words ? gs_bin_sorted_words(c, t->n, &pre, cam->width, cam->height,
-                                             static_cast<uint64_t*>(t->keys_sorted.p), cap, v.ranges.u(), K)
-                       : gs_bin_tiles_impl(c, t->n, &pre, cam->width, cam->height, t->keys_sorted.u(), cap,
-                                           v.ranges.u(), K, nullptr, nullptr, c->split_groups);
+        const uint32_t cap = (uint32_t)std::min<size_t>(t->keys_sorted.bytes / 8, 0xFFFFFFFFu);
+        int st = gs_bin_sorted_words(c, t->n, &pre, cam->width, cam->height, static_cast<uint64_t*>(t->keys_sorted.p),
+                                     cap, v.ranges.u(), K);
         if (st == GS_ERR_CAPACITY && *K > (long long)cap && attempt == 0) {
-            TR_TRY(t->keys_sorted.ensure((size_t)(*K + *K / 8 + 1024) * per));
+            TR_TRY(t->keys_sorted.ensure((size_t)(*K + *K / 8 + 1024) * 8));
             continue;
         }
         TR_TRY(st);
-        t->pair_stride = words ? 2 : 1;
+        t->pair_stride = 2;
         return GS_OK;
     }
     return gs_set_error(GS_ERR_CAPACITY, "trainer binning: pair buffer did not grow");
@@ -315,16 +321,16 @@ static int tr_forward(gs_trainer* t, gs::ViewBufs& v, const gs_camera* cam, cons
     const bool direct = (cam->width + 15) / 16 <= GS_BIN_MAX_TILES_XY && (cam->height + 15) / 16 <= GS_BIN_MAX_TILES_XY;
     if (direct && t->keys_sorted.bytes >= 4 && t->allow_async) {
         if (!t->k_pinned) {
-            // mapped + coherent: the scan kernel stores the count straight into it
-            hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&t->k_pinned), 8,
+            // mapped + coherent: the kernels store the pair and record counts straight into it
+            hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&t->k_pinned), 16,
                                          hipHostMallocMapped | hipHostMallocCoherent);
             if (e == hipSuccess) e = hipHostGetDevicePointer(reinterpret_cast<void**>(&t->k_pinned_dev), t->k_pinned, 0);
             if (e == hipSuccess) e = hipEventCreateWithFlags(&t->k_event, hipEventDisableTiming);
             if (e != hipSuccess) return gs_hip_status(e, "pinned pair count");
         }
         const uint32_t cap = (uint32_t)std::min<size_t>(t->keys_sorted.bytes / 4, 0xFFFFFFFFu);
-        TR_TRY(gs_bin_tiles_impl(c, t->n, &pre, cam->width, cam->height, t->keys_sorted.u(), cap, v.ranges.u(), nullptr,
-                                 t->k_pinned_dev, t->k_event, c->split_groups));
+        TR_TRY(gs_bin_prepare(c, t->n, &pre, cam->width, cam->height, nullptr, t->k_pinned_dev, t->k_event));
+        TR_TRY(gs_bin_finish(c, t->keys_sorted.u(), cap, v.ranges.u()));
         t->pair_stride = 1;
         *pending = true;
     } else {
@@ -333,23 +339,7 @@ static int tr_forward(gs_trainer* t, gs::ViewBufs& v, const gs_camera* cam, cons
     TR_TRY(tr_mark(t, GS_STAGE_BINNING, false));
     gs_pixel_state px{v.T_final.f(), v.n_contrib.i(), v.last.u()};
     TR_TRY(tr_mark(t, GS_STAGE_RASTER_FWD, true));
-    gsr::RasterSplit sp;
-    TR_TRY(gs_bin_split_info(c, &sp, nullptr));
-    if (t->pair_stride == 1 && sp.round == 1) {
-        // two rounds: render what the binning placed (the nearest depth groups),
-        // place the rest for the bins with unfinished tiles, resume those tiles
-        const size_t tiles = (size_t)((cam->width + 15) / 16) * ((cam->height + 15) / 16);
-        TR_TRY(v.split_flags.ensure(tiles * 4));
-        TR_TRY(v.split_rc.ensure((size_t)cam->width * cam->height * 12));
-        sp.tile_flag = v.split_flags.u();  // written by round 1 for every tile
-        sp.rc = v.split_rc.f();
-        TR_TRY(gs_raster_fwd_split(c, cam->width, cam->height, &pre, t->keys_sorted.u(), v.ranges.u(),
-                                   cfg->bg_color, v.image.f(), &px, &sp));
-        TR_TRY(gs_bin_place_rest(c, sp.tile_flag));
-        sp.round = 2;
-        TR_TRY(gs_raster_fwd_split(c, cam->width, cam->height, &pre, t->keys_sorted.u(), v.ranges.u(),
-                                   cfg->bg_color, v.image.f(), &px, &sp));
-    } else if (t->pair_stride == 1)
+    if (t->pair_stride == 1)
         TR_TRY(gs_raster_fwd(c, cam->width, cam->height, &pre, t->keys_sorted.u(), v.ranges.u(), cfg->bg_color,
                              v.image.f(), &px));
     else
@@ -365,16 +355,20 @@ static int tr_forward(gs_trainer* t, gs::ViewBufs& v, const gs_camera* cam, cons
 static int tr_pairs(gs_trainer* t, long long* K, bool* fits) {
     hipError_t e = hipEventSynchronize(t->k_event);
     if (e != hipSuccess) return gs_hip_status(e, "hipEventSynchronize");
-    *K = (long long)*static_cast<volatile unsigned long long*>(t->k_pinned);
+    const volatile unsigned long long* counts = t->k_pinned;
+    *K = (long long)counts[0];
     const size_t cap = t->keys_sorted.bytes / 4;
     *fits = (size_t)*K <= cap;
+    bool records_fit = true;  // if not, the lists and K are cut short: the redo counts again
+    TR_TRY(gs_bin_fits(t->ctx, *t->ctx->bin, counts[1], &records_fit));
+    *fits = *fits && records_fit;
     if (!*fits) {
         // the dropped pairs raised the context's overflow flag: clear it, grow
         void* sm = nullptr;
         TR_TRY(gs_small_get(t->ctx, &sm));
         e = launch_zero(static_cast<char*>(sm) + GS_SMALL_OVERFLOW, 4, t->ctx->stream);
         if (e != hipSuccess) return gs_hip_status(e, "zero kernel");
-        TR_TRY(t->keys_sorted.ensure((size_t)(*K + *K / 8 + 1024) * 4));
+        if ((size_t)*K > cap) TR_TRY(t->keys_sorted.ensure((size_t)(*K + *K / 8 + 1024) * 4));
     }
     return GS_OK;
 }

@@ -28,7 +28,6 @@ struct ViewBufs {
     DevBuf means2D, depths, conics, op2d, rgb, radii, tiles, offsets, ranges;
     DevBuf image, d_image, T_final, n_contrib, last, loss;
     DevBuf rg;  // screen-space gradients, one block: means2D (8 B/G), conics (12), rgb (12), opacities (4)
-    DevBuf split_flags, split_rc;  // two-round forward: tile and bin flags; per-pixel colour
     size_t rg_n = 0;
     gs_preprocessed pre();
     gs_raster_grads rgrads();
@@ -70,7 +69,7 @@ struct gs_trainer {
     gs::DevBuf keys, vals, keys_sorted, vals_sorted;
     int pair_stride = 1;  // uint32 entries per pair in keys_sorted: 1 (indices) or 2 (words)
     int fused_adam = 0;   // Adam applied inside the preprocess backward (gradients not written)
-    unsigned long long* k_pinned = nullptr;      // pair count of a pending binning (mapped pinned host memory)
+    unsigned long long* k_pinned = nullptr;      // pair and record counts of a pending binning (mapped pinned host memory)
     unsigned long long* k_pinned_dev = nullptr;  // its device address
     hipEvent_t k_event = nullptr;             // recorded after its copy
     bool allow_async = true;

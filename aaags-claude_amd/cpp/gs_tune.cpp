@@ -4,12 +4,10 @@
 // stage at a time over that knob's candidates (coordinate descent), timing
 // each candidate with HIP events on the context's stream (candidates
 // interleaved, median of `reps` runs each), and keeps the fastest:
-//   binning:         tiles per lane {1, 2, 4}, then group size {1024 .. 65536},
-//                    then the depth-sort digit width {4 .. 8};
+//   binning:         the depth-sort digit width {4 .. 8};
 //   raster forward:  LDS batch depth {64, 128, 256, 512};
-//   raster backward: LDS batch depth {64, 128, 256};
-//   forward:         depth groups placed before the first raster round
-//                    {0 (one round), 2, 4, 8, 16, 32}, on whole forward renders.
+//   raster backward: LDS batch depth {64, 128, 256}.
+// The whole forward is timed once with the chosen knobs.
 // Only forward, loss and backward stages run: the trainer's parameters and
 // optimizer state are untouched.
 #include <hip/hip_runtime.h>
@@ -110,10 +108,9 @@ extern "C" int gs_autotune(gs_trainer* t, const gs_camera* cam, const gs_render_
     gs_tuning res{};
     long long k2 = 0;
     auto bin = [&]() { return gs_bin_tiles(c, t->n, &pre, W, H, t->keys_sorted.u(), cap, v.ranges.u(), &k2); };
-    TU_TRY(pick(c, tm, reps, {1, 2, 4}, [&](int x) { return gs_ctx_set_binning(c, 0, x); }, bin,
-                &res.bin_tiles_per_lane, &res.binning_ms));
-    TU_TRY(pick(c, tm, reps, {1024, 2048, 4096, 8192, 16384, 32768, 65536}, [&](int x) { return gs_ctx_set_binning(c, x, 0); },
-                bin, &res.bin_group, &res.binning_ms));
+    res.bin_tiles_per_lane = c->bin_tpl;  // knobs without effect, reported unchanged
+    res.bin_group = c->bin_chunk;
+    res.split_groups = c->split_groups;
     TU_TRY(pick(c, tm, reps, {4, 5, 6, 7, 8}, [&](int x) { return gs_ctx_set_tuning(c, x, 0, 0); }, bin,
                 &res.radix_bits, &res.binning_ms));
     TU_TRY(bin());  // the pair lists of the chosen setting
@@ -133,16 +130,10 @@ extern "C" int gs_autotune(gs_trainer* t, const gs_camera* cam, const gs_render_
     TU_TRY(pick(c, tm, reps, {64, 128, 256}, [&](int x) { return gs_ctx_set_tuning(c, 0, 0, x); }, bwd,
                 &res.raster_bwd_batch, &res.raster_bwd_ms));
     res.persistent_per_cu = c->persistent_per_cu;
-    // the two-round forward: groups placed before the first raster round, on
-    // the trainer's whole forward with the knobs chosen above
     long long k3 = 0;
-    auto render = [&]() { return gs_trainer_render(t, cam, cfg, &k3); };
-    TU_TRY(pick(c, tm, reps, {0, 16, 32, 64, 128},
-                [&](int x) {
-                    c->split_groups = x;
-                    return GS_OK;
-                },
-                render, &res.split_groups, &res.forward_ms));
+    int unused = 0;
+    TU_TRY(pick(c, tm, reps, {0}, [](int) { return GS_OK; }, [&]() { return gs_trainer_render(t, cam, cfg, &k3); },
+                &unused, &res.forward_ms));
     if (hipStreamSynchronize(c->stream) != hipSuccess) return gs_set_error(GS_ERR_HIP, "hipStreamSynchronize");
     if (out) *out = res;
     return GS_OK;

@@ -2,6 +2,7 @@
 // workspace, and kernel launches on the context stream.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <cstdio>
@@ -87,21 +88,14 @@ extern "C" int gs_ctx_create(int device, void* stream, gs_ctx** out) {
     return GS_OK;
 }
 
-// The split a gs_bin_tiles_impl call left pending: the placement arguments
-// for the remaining depth groups and what the forward raster needs.
-struct BinSplit {
-    bool pending = false;
-    gsb::BinArgs a{};
-    int tpl = 1, bins = 0, C = 0, split = 0, gx = 0, gy = 0;
-};
-
 extern "C" int gs_ctx_destroy(gs_ctx* c) {
     if (!c) return GS_OK;
     (void)hipSetDevice(c->device);
     if (c->ws) (void)hipFree(c->ws);
     if (c->ws2) (void)hipFree(c->ws2);
     if (c->small) (void)hipFree(c->small);
-    delete static_cast<BinSplit*>(c->bin_split);
+    if (c->coarse) (void)hipFree(c->coarse);
+    delete c->bin;
     delete c;
     return GS_OK;
 }
@@ -160,7 +154,10 @@ static int grow(gs_ctx* c, void** buf, size_t* have, size_t bytes, void** out) {
 }
 
 int gs_ws_get(gs_ctx* c, size_t bytes, void** out) { return grow(c, &c->ws, &c->ws_bytes, bytes, out); }
-int gs_ws2_get(gs_ctx* c, size_t bytes, void** out) { return grow(c, &c->ws2, &c->ws2_bytes, bytes, out); }
+int gs_ws2_get(gs_ctx* c, size_t bytes, void** out) {
+    c->bin_pending = false;  // a prepared binning lives in this workspace
+    return grow(c, &c->ws2, &c->ws2_bytes, bytes, out);
+}
 
 // Small fixed scratch: scan partials, overflow flags, loss partials.
 int gs_small_get(gs_ctx* c, void** out) {
@@ -459,10 +456,8 @@ extern "C" int gs_bin_sorted_words(gs_ctx* c, int n, const gs_preprocessed* pre,
     return GS_OK;
 }
 
-// Direct-placement binning knobs (0 keeps a value): Gaussians per group
-// (larger groups shrink the (tile, group) table and lengthen each block's walk
-// and its contiguous output runs) and tiles per lane (bins of 8 x 8*tpl tiles;
-// larger bins mean fewer walks over the records, more work per visit).
+// Binning knobs (0 keeps a value), checked and kept for stored tunings; the
+// binning's layout follows the sizes (bin_layout).
 extern "C" int gs_ctx_set_binning(gs_ctx* c, int gaussians_per_group, int tiles_per_lane) {
     GS_CHECK_ARG(c != nullptr, "null context");
     if (gaussians_per_group) {
@@ -504,164 +499,153 @@ extern "C" int gs_ctx_apply_tuning(gs_ctx* c, const gs_tuning* t) {
     return GS_OK;
 }
 
-// gs_bin_tiles, and its form for drivers that keep the GPU busy: with
-// total_async (the device address of mapped, coherent pinned host memory) the
-// scan writes the pair count there without a host wait (`ev_total` is
-// recorded after the scan), the placement runs with
-// the given capacity whatever the count, pairs past it are dropped (overflow
-// flag) and the ranges are clamped to it; the caller compares the count with
-// the capacity before using the results.
-int gs_bin_tiles_impl(gs_ctx* c, int n, const gs_preprocessed* pre, int width, int height, uint32_t* values,
-                      uint32_t capacity, uint32_t* ranges, long long* total_host, unsigned long long* total_async,
-                      hipEvent_t ev_total, int split) {
+// Room for at least `records` bin records.
+static int coarse_get(gs_ctx* c, size_t records, gsb::BinArgs& a) {
+    const size_t each = bin_record_bytes(a);
+    int st = grow(c, &c->coarse, &c->coarse_bytes, records * each, &a.coarse);
+    if (st) return st;
+    a.coarse_cap = (uint32_t)std::min<size_t>(c->coarse_bytes / each, 0xFFFFFFFFu);
+    return GS_OK;
+}
+
+int gs_bin_fits(gs_ctx* c, const gsb::BinArgs& a, unsigned long long records, bool* fits) {
+    *fits = records <= a.coarse_cap;
+    if (*fits) return GS_OK;
+    if (records > 0xFFFFFFFFull)
+        return gs_set_error(GS_ERR_CAPACITY, "binning: %llu bin records exceed 2^32-1", records);
+    gsb::BinArgs grown = a;
+    return coarse_get(c, (size_t)records, grown);
+}
+
+// First guess for the record buffer, in records per Gaussian (6 at 1M
+// Gaussians and 1080p; a view that needs more grows it once).
+constexpr size_t kRecordsPerGaussian = 8;
+
+int gs_bin_count(gs_ctx* c, gsb::BinArgs& a, unsigned long long* pairs) {
+    void* sm;
+    int st = gs_small_get(c, &sm);
+    if (st) return st;
+    // {pairs, records} side by side: one copy reads both
+    unsigned long long* counts = reinterpret_cast<unsigned long long*>(static_cast<char*>(sm) + GS_SMALL_TOTAL64);
+    a.overflow = reinterpret_cast<uint32_t*>(static_cast<char*>(sm) + GS_SMALL_OVERFLOW);
+    if ((st = coarse_get(c, (size_t)a.V * a.N * kRecordsPerGaussian, a))) return st;
+    unsigned long long got[2] = {0, 0};
+    for (int attempt = 0;; attempt++) {
+        GS_HIP(launch_bin_lists(a, c->stream, counts + 1, nullptr, counts, attempt > 0), "binning kernels");
+        GS_HIP(hipMemcpyAsync(got, counts, 16, hipMemcpyDeviceToHost, c->stream), "hipMemcpyAsync(total)");
+        GS_HIP(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+        if (got[1] <= a.coarse_cap) break;
+        bool fits;
+        if ((st = gs_bin_fits(c, a, got[1], &fits))) return st;
+        if (attempt > 0) return gs_set_error(GS_ERR_CAPACITY, "binning: the record buffer did not grow");
+        if ((st = coarse_get(c, (size_t)got[1], a))) return st;
+        GS_HIP(launch_zero(a.overflow, 4, c->stream), "zero kernel");  // raised by the records that did not fit
+    }
+    *pairs = got[0];
+    return GS_OK;
+}
+
+int gs_bin_prepare(gs_ctx* c, int n, const gs_preprocessed* pre, int width, int height, long long* pairs,
+                   unsigned long long* host_counts, hipEvent_t ev_total) {
     GS_CHECK_ARG(c != nullptr, "null context");
     GS_CHECK_ARG(width > 0 && height > 0, "bad image size");
     GS_CHECK_ARG(n >= 0, "negative count");
-    GS_CHECK_ARG(ranges != nullptr, "null tile ranges");
     int st = check_pre(pre, true);
     if (st) return st;
     const int gx = (width + 15) / 16, gy = (height + 15) / 16;
-    const int num_tiles = gx * gy;
     if (gx > GS_BIN_MAX_TILES_XY || gy > GS_BIN_MAX_TILES_XY)
         return gs_set_error(GS_ERR_UNSUPPORTED, "gs_bin_tiles: %d x %d tiles exceed %d per side (use gs_bin_sorted_words)",
                             gx, gy, GS_BIN_MAX_TILES_XY);
-    GS_CHECK_ARG(aligned(values, 16) || values == nullptr, "values must be 16-byte aligned");
-    if (n == 0) {
-        GS_HIP(launch_zero(ranges, (size_t)num_tiles * 8, c->stream), "zero kernel");
-        if (total_host) *total_host = 0;
+    if (!c->bin) c->bin = new gsb::BinArgs();
+    gsb::BinArgs& a = *c->bin;
+    a = gsb::BinArgs{};
+    a.V = 1;
+    a.N = n;
+    a.total_tiles = gx * gy;
+    a.side = bin_side(gx, gy);
+    a.max_bins = bin_count_of_view(a.side, gx, gy);
+    a.NB = (uint32_t)a.max_bins;
+    a.view0 = make_int4(gx, gy, 0, 0);
+    c->bin_pending = true;
+    if (n == 0) {  // the ranges are cleared by gs_bin_finish
+        if (pairs) *pairs = 0;
         return GS_OK;
     }
-    void* sm;
-    if ((st = gs_small_get(c, &sm))) return st;
-    uint32_t* ovf = reinterpret_cast<uint32_t*>(static_cast<char*>(sm) + GS_SMALL_OVERFLOW);
+    c->bin_pending = false;
+    bin_layout(a);
+    GS_CHECK_ARG(a.table2_len < 0xFFFFFFFFull, "binning table too large");
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
     const size_t un = (size_t)n;
-    // with a split, the first `split` groups are small (the nearest
-    // Gaussians, placed before the first raster round: small groups give that
-    // placement more blocks), the rest have the configured size
-    const int G = c->bin_chunk;
-    const int G1 = G < GS_SPLIT_GROUP ? G : GS_SPLIT_GROUP;
-    const int S = (split > 0 && (long long)split * G1 < n) ? split : 0;
-    const int C = S + (n - S * G1 + G - 1) / G;
-    const size_t L = (size_t)C * num_tiles + 1;
-    GS_CHECK_ARG(L < 0xFFFFFFFFull, "binning table too large");
-    const size_t np = scan_partials_needed((uint32_t)L) + 1;
     void* ws2;
-    if ((st = gs_ws2_get(c, 2 * al(un * 8) + al(un * 8) + al(un * 4) + radix_workspace_bytes((uint32_t)n, 8) +
-                                2 * al(L * 4) + al(np * 8),
+    if ((st = gs_ws2_get(c, 2 * al(un * 8) + al(un * 4) + radix_workspace_bytes((uint32_t)n, c->radix_bits) +
+                                bin_workspace_bytes(a),
                          &ws2)))
         return st;
     char* w = static_cast<char*>(ws2);
     uint64_t* dkeys = reinterpret_cast<uint64_t*>(w); w += al(un * 8);    // index << 32 | depth key
     uint64_t* dkeys_s = reinterpret_cast<uint64_t*>(w); w += al(un * 8);  // the same, in depth order
-    uint2* rects = reinterpret_cast<uint2*>(w); w += al(un * 8);
     uint32_t* rect_idx = reinterpret_cast<uint32_t*>(w); w += al(un * 4);  // packed rectangles, index order
-    uint32_t* table = reinterpret_cast<uint32_t*>(w); w += al(L * 4);
-    uint32_t* scanned = reinterpret_cast<uint32_t*>(w); w += al(L * 4);
-    unsigned long long* partial = reinterpret_cast<unsigned long long*>(w); w += al(np * 8);
     void* dsort_ws = w;
+    bin_carve(a, w + radix_workspace_bytes((uint32_t)n, c->radix_bits));
     GS_HIP(launch_depth_words(n, pre->depths, pre->radii, dkeys, c->stream, pre->means2D, gx, gy, rect_idx),
            "depth keys kernel");
     GS_HIP(launch_radix_sort_bits(dkeys, nullptr, dkeys_s, nullptr, (uint32_t)n, 0, 32, c->radix_bits, dsort_ws,
                                   c->stream, nullptr),
            "depth sort");
-    gsb::BinArgs a{};
-    a.V = 1;
-    a.N = n;
-    a.C = C;
-    a.G = G;
-    a.S = S;
-    a.G1 = G1;
     a.sidx = reinterpret_cast<const uint32_t*>(dkeys_s) + 1;  // the index words
     a.sidx_stride = 2;
-    a.means2D = reinterpret_cast<const float2*>(pre->means2D);
-    a.radii = pre->radii;
-    a.views = nullptr;
-    a.view0 = make_int4(gx, gy, 0, 0);
-    a.vblock0 = nullptr;
-    a.table = table;
-    a.table_len = L;
-    a.rects = rects;
-    a.out = values;
-    a.capacity = capacity;
-    a.overflow = ovf;
-    a.diff_len = (gx + 1) * (gy + 1);
     a.rect_idx = rect_idx;
-    unsigned long long* total64 = reinterpret_cast<unsigned long long*>(static_cast<char*>(sm) + GS_SMALL_TOTAL64);
-    const int blocks = bin_blocks(C, gx, gy, c->bin_tpl);
-    GS_HIP(launch_bin_count(a, blocks, c->bin_tpl, c->stream), "binning count kernel");
-    // with a split, only the first `split` depth groups are placed now (blocks
-    // are numbered group-major: group c's blocks are c * bins .. c * bins + bins - 1)
-    if (!c->bin_split) c->bin_split = new BinSplit();
-    BinSplit* bs = static_cast<BinSplit*>(c->bin_split);
-    bs->pending = false;
-    const int bins = blocks / C;
-    int place_blocks = blocks;
-    if (S > 0) {
-        place_blocks = S * bins;
-        bs->pending = true;
-        bs->tpl = c->bin_tpl;
-        bs->bins = bins;
-        bs->C = C;
-        bs->split = S;
-        bs->gx = gx;
-        bs->gy = gy;
-    }
-    // asynchronous: the scan writes the pair count straight into the caller's
-    // mapped host memory, and the event marks when it is there
-    GS_HIP(launch_scan_u32_exclusive(table, (uint32_t)L, scanned, partial, c->stream, nullptr,
-                                     total_async ? total_async : total64),
-           "binning scan");
-    a.table = scanned;
-    bs->a = a;
-    if (total_async) {
-        GS_CHECK_ARG(values != nullptr && capacity > 0, "null values buffer");
+    if (host_counts) {
+        void* sm;
+        if ((st = gs_small_get(c, &sm))) return st;
+        a.overflow = reinterpret_cast<uint32_t*>(static_cast<char*>(sm) + GS_SMALL_OVERFLOW);
+        if ((st = coarse_get(c, un * kRecordsPerGaussian, a))) return st;
+        GS_HIP(launch_bin_lists(a, c->stream, host_counts + 1, nullptr, host_counts), "binning kernels");
         if (ev_total) GS_HIP(hipEventRecord(ev_total, c->stream), "hipEventRecord");
-        GS_HIP(launch_bin_place(a, place_blocks, c->bin_tpl, c->stream), "binning place kernel");
-        GS_HIP(launch_bin_ranges(a, scanned, (uint32_t)num_tiles, ranges, c->stream), "binning ranges kernel");
+    } else {
+        unsigned long long K = 0;
+        if ((st = gs_bin_count(c, a, &K))) return st;
+        if (pairs) *pairs = (long long)K;
+    }
+    c->bin_pending = true;
+    return GS_OK;
+}
+
+int gs_bin_finish(gs_ctx* c, uint32_t* values, uint32_t capacity, uint32_t* ranges) {
+    GS_CHECK_ARG(c != nullptr, "null context");
+    GS_CHECK_ARG(c->bin_pending, "no binning pending");
+    GS_CHECK_ARG(ranges != nullptr, "null tile ranges");
+    GS_CHECK_ARG(aligned(values, 16) || values == nullptr, "values must be 16-byte aligned");
+    c->bin_pending = false;
+    gsb::BinArgs& a = *c->bin;
+    if (a.N == 0) {
+        GS_HIP(launch_zero(ranges, (size_t)a.total_tiles * 8, c->stream), "zero kernel");
         return GS_OK;
     }
-    unsigned long long K = 0;
-    GS_HIP(hipMemcpyAsync(&K, total64, 8, hipMemcpyDeviceToHost, c->stream), "hipMemcpyAsync(total)");
-    GS_HIP(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
-    if (total_host) *total_host = (long long)K;
-    if (K > capacity) return gs_set_error(GS_ERR_CAPACITY, "gs_bin_tiles: %llu pairs exceed capacity %u", K, capacity);
-    if (K > 0) {
-        GS_CHECK_ARG(values != nullptr, "null values buffer");
-        GS_HIP(launch_bin_place(a, place_blocks, c->bin_tpl, c->stream), "binning place kernel");
-    } else {
-        bs->pending = false;
-    }
-    GS_HIP(launch_bin_ranges(a, scanned, (uint32_t)num_tiles, ranges, c->stream), "binning ranges kernel");
+    a.out = values;
+    a.capacity = values ? capacity : 0u;
+    if (a.capacity > 0u) GS_HIP(launch_bin_place(a, c->stream), "binning place kernel");
+    GS_HIP(launch_bin_ranges(a, ranges, c->stream), "binning ranges kernel");
     return GS_OK;
 }
 
 extern "C" int gs_bin_tiles(gs_ctx* c, int n, const gs_preprocessed* pre, int width, int height, uint32_t* values,
                             uint32_t capacity, uint32_t* ranges, long long* total_host) {
-    return gs_bin_tiles_impl(c, n, pre, width, height, values, capacity, ranges, total_host, nullptr, nullptr);
-}
-
-int gs_bin_split_info(gs_ctx* c, gsr::RasterSplit* sp, int* num_bins) {
-    GS_CHECK_ARG(c && sp, "null argument");
-    *sp = gsr::RasterSplit{};
-    const BinSplit* bs = static_cast<const BinSplit*>(c->bin_split);
-    if (!bs || !bs->pending) return GS_OK;
-    sp->scanned = bs->a.table;
-    sp->C = bs->C;
-    sp->g1 = bs->split;
-    sp->round = 1;
-    if (num_bins) *num_bins = bs->bins;
-    return GS_OK;
-}
-
-int gs_bin_place_rest(gs_ctx* c, const uint32_t* tile_gate) {
-    GS_CHECK_ARG(c != nullptr, "null context");
-    BinSplit* bs = static_cast<BinSplit*>(c->bin_split);
-    GS_CHECK_ARG(bs && bs->pending, "no split binning pending");
-    GS_HIP(launch_bin_place(bs->a, (bs->C - bs->split) * bs->bins, bs->tpl, c->stream, bs->split * bs->bins, tile_gate),
-           "binning place kernel (remaining groups)");
-    bs->pending = false;
-    return GS_OK;
+    GS_CHECK_ARG(ranges != nullptr, "null tile ranges");
+    GS_CHECK_ARG(aligned(values, 16) || values == nullptr, "values must be 16-byte aligned");
+    long long K = 0;
+    int st = gs_bin_prepare(c, n, pre, width, height, &K, nullptr, nullptr);
+    if (st) return st;
+    if (total_host) *total_host = K;
+    if (K > (long long)capacity) {
+        c->bin_pending = false;
+        return gs_set_error(GS_ERR_CAPACITY, "gs_bin_tiles: %lld pairs exceed capacity %u", K, capacity);
+    }
+    if (K > 0 && !values) {
+        c->bin_pending = false;
+        return gs_set_error(GS_ERR_INVALID, "null values buffer");
+    }
+    return gs_bin_finish(c, values, capacity, ranges);
 }
 
 static gsr::RasterArgs raster_args(int width, int height, const gs_preprocessed* pre, const uint32_t* values,
@@ -685,7 +669,7 @@ static gsr::RasterArgs raster_args(int width, int height, const gs_preprocessed*
 
 static int raster_fwd_impl(gs_ctx* c, int width, int height, const gs_preprocessed* pre, const uint32_t* values,
                            int vstride, const uint32_t* ranges, const float bg[3], float* image,
-                           const gs_pixel_state* px, const gsr::RasterSplit* sp = nullptr) {
+                           const gs_pixel_state* px) {
     GS_CHECK_ARG(c != nullptr, "null context");
     GS_CHECK_ARG(width > 0 && height > 0, "bad image size");
     int st = check_pre(pre, false);
@@ -694,16 +678,9 @@ static int raster_fwd_impl(gs_ctx* c, int width, int height, const gs_preprocess
     int tiles = ((width + 15) / 16) * ((height + 15) / 16);
     gsr::RasterArgs a = raster_args(width, height, pre, values, ranges, bg, vstride);
     GS_HIP(launch_raster_fwd(a, tiles, c->raster_batch, image, px ? px->T_final : nullptr,
-                             px ? px->n_contrib : nullptr, px ? px->last_contrib : nullptr, c->stream, sp),
+                             px ? px->n_contrib : nullptr, px ? px->last_contrib : nullptr, c->stream),
            "raster forward kernel");
     return GS_OK;
-}
-
-int gs_raster_fwd_split(gs_ctx* c, int width, int height, const gs_preprocessed* pre, const uint32_t* values,
-                        const uint32_t* ranges, const float bg[3], float* image, const gs_pixel_state* px,
-                        const gsr::RasterSplit* sp) {
-    GS_CHECK_ARG(px && px->T_final && px->n_contrib && px->last_contrib, "a split forward needs the pixel state");
-    return raster_fwd_impl(c, width, height, pre, values, 1, ranges, bg, image, px, sp);
 }
 
 extern "C" int gs_raster_fwd(gs_ctx* c, int width, int height, const gs_preprocessed* pre, const uint32_t* values,

@@ -416,21 +416,6 @@ struct RasterArgs {
     float bg0, bg1, bg2;
     int vstride;  // 1: uint32 value array; 2: low words of tile<<32|index pairs
 };
-// Forward raster in two rounds over a pair list placed in two parts (one
-// view): the binning placed only the first g1 depth groups of every tile's
-// list; round 1 renders each tile up to where group g1 begins, writes every
-// tile's flag (1: not finished there) and saves the pixels' state of the
-// unfinished ones; the rest of the list is then placed for bins with a
-// flagged tile only, and round 2 resumes the flagged tiles.  round 0: one
-// pass (no split).
-struct RasterSplit {
-    const uint32_t* scanned;  // the scanned binning table: slot of (tile, group)'s first pair
-    int C, g1;                // groups per view; groups placed before round 1 (g1 < C)
-    uint32_t* tile_flag;      // per tile, written by round 1
-    float* rc;                // per pixel: accumulated colour (3 floats) of an unfinished tile
-    int round;                // 0, 1 or 2
-};
-
 struct GradArgs {
     float2* d_means2D;
     float* d_conics;
@@ -471,26 +456,38 @@ struct MultiGrads {  // view-major [V][N]
 }  // namespace gsr
 
 namespace gsb {
-// Direct-placement binning over V views of N Gaussians each (k_bin.hip).
+// Direct-placement binning over V views of N Gaussians each (k_bin.hip): bins
+// of side x side tiles, the Gaussians in chunks (level 1) and groups of chunks
+// (level 2).
 struct BinArgs {
     int V, N;
-    int C, G;               // groups per view; Gaussians per group after the first S
-    int S, G1;              // the first S groups hold G1 Gaussians each (0: none)
-    const uint32_t* sidx;   // [V*N]: each view's Gaussian indices in depth order, sidx_stride apart
+    int total_tiles;        // over all views
+    int side;               // tiles per bin side, 4 or 8 (bin_side)
+    uint32_t NB;            // bins over all views
+    int max_bins;           // bins of the largest view
+    int CH, C1;             // Gaussians per chunk, chunks per view (bin_layout)
+    int GC, C2;             // chunks per group, groups per view (bin_layout)
+    const uint32_t* sidx;   // [V*N]: each view's Gaussian indices in order, sidx_stride apart (null: index order)
     int sidx_stride;        // 1: an index array; 2: the high words of sorted index << 32 | key words
     const float2* means2D;  // view-major [V][N]
     const int* radii;       // [V][N]
-    const int4* views;      // per view: (tiles per row, tile rows, table offset, first global tile)
-    int4 view0;             // used instead when views == nullptr (one view)
-    const int* vblock0;     // per view: first block (V + 1 entries); nullptr for one view
-    uint32_t* table;        // count: per-(view, tile, group) counts; place: their exclusive scan
-    size_t table_len;       // sum over views of tiles * C, plus one trailing entry
-    uint2* rects;           // [V*N] scratch: depth-ordered (x0|x1<<8|y0<<16|y1<<24, index)
-    uint32_t* out;          // place: pair values (Gaussian index); 16-byte aligned
-    uint32_t capacity;
-    uint32_t* overflow;
-    int diff_len;           // max over views of (tiles per row + 1) * (tile rows + 1); 0: no LDS count
     const uint32_t* rect_idx;  // optional [V][N]: packed rectangles by Gaussian index (else from means2D, radii)
+    const int4* views;      // per view: (tiles per row, tile rows, first bin, first global tile)
+    int4 view0;             // used instead when views == nullptr (one view)
+    // workspace (bin_carve)
+    uint2* rects;           // [V*N]: ordered (x0 | x1 << 8 | y0 << 16 | y1 << 24, index)
+    uint32_t* table1;       // [C1][NB]: counts, then their scan over the chunks
+    size_t table1_len;
+    uint32_t *tot, *start;  // per bin: records; first record (NB + 1 entries)
+    uint32_t *table2, *scanned;  // (tile, group): counts; their exclusive scan (one trailing entry)
+    size_t table2_len;
+    unsigned long long* partial;
+    // the bins' records (index, tile mask) and the pair values
+    void* coarse;           // 8 bytes per record with bins of side 4, 16 with side 8
+    uint32_t coarse_cap;    // records
+    uint32_t* out;          // Gaussian index per pair; 16-byte aligned
+    uint32_t capacity;
+    uint32_t* overflow;     // raised when records or pairs outgrow their buffer
 };
 }  // namespace gsb
 

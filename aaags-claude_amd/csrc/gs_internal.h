@@ -10,7 +10,7 @@
 #include "gs_hip.h"
 
 namespace gsd { struct CamArgs; }
-namespace gsr { struct RasterArgs; struct RasterSplit; struct GradArgs; struct MultiRaster; struct MultiPix; struct MultiGrads; }
+namespace gsr { struct RasterArgs; struct GradArgs; struct MultiRaster; struct MultiPix; struct MultiGrads; }
 namespace gso { struct AdamArgs; struct AdamDev; }
 namespace gsb { struct BinArgs; }
 
@@ -31,13 +31,16 @@ struct gs_ctx {
     int radix_bits = 8;
     int raster_batch = 256;
     int raster_bwd_batch = 256;
-    int bin_chunk = 4096;   // Gaussians per group in direct-placement binning
-#define GS_SPLIT_GROUP 1024     // Gaussians per group of the part placed before the first raster round
-    int bin_tpl = 1;        // tiles per lane (bin = 8 x 8*tpl tiles)
+    // Knobs of earlier binning kernels (Gaussians per group, tiles per lane):
+    // kept for stored tunings, without effect (the layout follows the sizes).
+    int bin_chunk = 4096;
+    int bin_tpl = 1;
     int persistent_per_cu = 6;  // batched raster: persistent groups per CU (0: one group per tile)
-    int split_groups = 64;      // trainer forward: groups of GS_SPLIT_GROUP Gaussians placed before the
-                                // first raster round (0: one round)
-    void* bin_split = nullptr;  // the split left pending by the last gs_bin_tiles_impl (BinSplit, capi.hip)
+    int split_groups = 64;      // likewise: the forward no longer runs in two rounds
+    void* coarse = nullptr;     // the binning's bin records
+    size_t coarse_bytes = 0;
+    gsb::BinArgs* bin = nullptr;  // the binning that gs_bin_begin left for gs_bin_place
+    bool bin_pending = false;
 };
 
 int gs_set_error(int code, const char* fmt, ...);
@@ -51,19 +54,24 @@ int gs_tile_key_bits(int num_tiles);
 extern "C" int gs_ctx_set_tuning(gs_ctx* c, int radix_bits, int raster_batch, int raster_bwd_batch);
 extern "C" int gs_ctx_reserve(gs_ctx* c, size_t bytes);
 extern "C" int gs_ctx_set_binning(gs_ctx* c, int gaussians_per_group, int tiles_per_lane);
-int gs_bin_tiles_impl(gs_ctx* c, int n, const gs_preprocessed* pre, int width, int height, uint32_t* values,
-                      uint32_t capacity, uint32_t* ranges, long long* total_host, unsigned long long* total_async,
-                      hipEvent_t ev_total, int split = 0);
-// After gs_bin_tiles_impl with 0 < split < groups, which placed only the
-// first `split` depth groups: the description of that split for the forward
-// raster (tile_flag and rc left to the caller), or sp->round = 0 when nothing
-// is pending; then the placement of the remaining groups for the bins with a
-// tile whose gate word is nonzero.
-int gs_bin_split_info(gs_ctx* c, gsr::RasterSplit* sp, int* num_bins);
-int gs_bin_place_rest(gs_ctx* c, const uint32_t* tile_gate);
-int gs_raster_fwd_split(gs_ctx* c, int width, int height, const gs_preprocessed* pre, const uint32_t* values,
-                        const uint32_t* ranges, const float bg[3], float* image, const gs_pixel_state* px,
-                        const gsr::RasterSplit* sp);
+// Direct-placement binning of one view.  Queues everything up to the pair
+// count, with the current capacity for bin records; then, either
+//  - host_counts (mapped, coherent pinned memory, device address) set: the
+//    kernels write {pairs, records} there, ev_total is recorded after them,
+//    and the caller compares both with the capacities before using results
+//    (gs_bin_fits); or
+//  - host_counts null: waits, grows the record buffer and repeats what needs it
+//    if the records did not fit, and returns the count in *pairs.
+int gs_bin_prepare(gs_ctx* c, int n, const gs_preprocessed* pre, int width, int height, long long* pairs,
+                   unsigned long long* host_counts, hipEvent_t ev_total);
+// Places the prepared pairs and writes the ranges; pairs past the capacity
+// are dropped (overflow flag) and the ranges clamped to it.
+int gs_bin_finish(gs_ctx* c, uint32_t* values, uint32_t capacity, uint32_t* ranges);
+// The same two halves over prepared arguments (order, sizes, views, rectangles
+// or means set; the workspace carved), for the eval_3D binning.
+int gs_bin_count(gs_ctx* c, gsb::BinArgs& a, unsigned long long* pairs);
+// Whether `records` bin records fit the context's buffer; grows it if not.
+int gs_bin_fits(gs_ctx* c, const gsb::BinArgs& a, unsigned long long records, bool* fits);
 extern "C" int gs_check_overflow(gs_ctx* c, int* overflowed);
 
 // kernel launchers
@@ -97,8 +105,7 @@ hipError_t launch_duplicate_ranked(int n, const uint32_t* order, const float* me
                                    const uint32_t* offsets, int gx, int gy, uint64_t* words, uint32_t capacity,
                                    uint32_t* overflow, hipStream_t s);
 hipError_t launch_raster_fwd(const gsr::RasterArgs& a, int num_tiles, int batch, float* img, float* T_final,
-                             int* n_contrib, uint32_t* last_contrib, hipStream_t s,
-                             const gsr::RasterSplit* split = nullptr);
+                             int* n_contrib, uint32_t* last_contrib, hipStream_t s);
 hipError_t launch_raster_bwd(const gsr::RasterArgs& a, int num_tiles, int batch, const float* T_final,
                              const uint32_t* last_contrib, const float* d_image, const gsr::GradArgs& g,
                              hipStream_t s);
@@ -128,12 +135,20 @@ hipError_t launch_duplicate_multi(uint32_t total, int N, const uint64_t* skeys, 
                                   uint64_t* words, uint32_t capacity, uint32_t* overflow, hipStream_t s);
 // direct-placement binning (k_bin.hip); larger views use the word sort
 constexpr int GS_BIN_MAX_TILES_XY = 255;  // tiles per row and per column (4080 pixels)
-int bin_blocks(int C, int gx, int gy, int tpl);
-hipError_t launch_bin_count(const gsb::BinArgs& a, int blocks, int tpl, hipStream_t s);
-hipError_t launch_bin_place(const gsb::BinArgs& a, int blocks, int tpl, hipStream_t s, int block0 = 0,
-                            const uint32_t* gate = nullptr);
-hipError_t launch_bin_ranges(const gsb::BinArgs& a, const uint32_t* scanned, uint32_t total_tiles, uint32_t* ranges,
-                             hipStream_t s);
+constexpr int GS_BIN_MAX_BINS = 1024;     // bins per view
+int bin_side(int max_gx, int max_gy);     // tiles per bin side for views of at most this many tiles
+int bin_count_of_view(int side, int gx, int gy);
+size_t bin_record_bytes(const gsb::BinArgs& a);
+void bin_layout(gsb::BinArgs& a);  // V, N, NB, total_tiles set: chunks, groups and table lengths
+size_t bin_workspace_bytes(const gsb::BinArgs& a);
+void bin_carve(gsb::BinArgs& a, void* workspace);
+// Bin records, tile counts and their scan.  records (device or mapped host):
+// the record count; total32 / total64 (optional): the pair count.  counted:
+// repeat after the record buffer grew (the bins' starts are there already).
+hipError_t launch_bin_lists(const gsb::BinArgs& a, hipStream_t s, unsigned long long* records, uint32_t* total32,
+                            unsigned long long* total64, bool counted = false);
+hipError_t launch_bin_place(const gsb::BinArgs& a, hipStream_t s);
+hipError_t launch_bin_ranges(const gsb::BinArgs& a, uint32_t* ranges, hipStream_t s);
 // total32 / total64 (optional, device): the sum of all n inputs
 hipError_t launch_scan_u32_exclusive(const uint32_t* in, uint32_t n, uint32_t* out, unsigned long long* partial,
                                      hipStream_t s, uint32_t* total32 = nullptr, unsigned long long* total64 = nullptr);

@@ -764,11 +764,6 @@ static Cam3 make_cam3(const gs_camera* cam, const gs_render_cfg* cfg, int model_
 constexpr int TS_THREADS = 1024, TS_ITEMS = 16, TS_WAVES = TS_THREADS / 64;
 constexpr int TS_CAP = TS_THREADS * TS_ITEMS;  // 16384 pairs per tile
 
-__global__ __launch_bounds__(256) void iota_kernel(uint32_t n, uint32_t* __restrict__ out) {
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (i < n) out[i] = i;
-}
-
 // A pair key's inputs per Gaussian in one 64-byte line: cov3D_inv (6),
 // mean_offset (3), depth, so that a pair's key costs three 16-byte loads of
 // one cache line instead of ten loads from three arrays.
@@ -1050,27 +1045,29 @@ extern "C" int gs_bin_tiles_3d(gs_ctx* c, int n, const gs_preprocessed* pre, con
     void* sm;
     int st = gs_small_get(c, &sm);
     if (st) return st;
-    uint32_t* ovf = reinterpret_cast<uint32_t*>(static_cast<char*>(sm) + GS_SMALL_OVERFLOW);
-    unsigned long long* total64 = reinterpret_cast<unsigned long long*>(static_cast<char*>(sm) + GS_SMALL_TOTAL64);
     auto alg = [](size_t x) { return (x + 255) & ~(size_t)255; };
-    // Gaussian-sized scratch: index order, rectangles, the (tile, group) table
-    // and its scan, the tiles' rays, the long lists' counts and offsets
     const size_t un = (size_t)n;
-    const int G = c->bin_chunk;
-    const int C = (n + G - 1) / G;
-    const size_t L = (size_t)C * num_tiles + 1;
-    G3_ARG(L < 0xFFFFFFFFull, "binning table too large");
-    const size_t np = scan_partials_needed((uint32_t)std::max<size_t>(L, (size_t)num_tiles + 1)) + 1;
+    gsb::BinArgs a{};
+    a.V = 1;
+    a.N = n;
+    a.total_tiles = num_tiles;
+    a.side = bin_side(k.gx, k.gy);
+    a.max_bins = bin_count_of_view(a.side, k.gx, k.gy);
+    a.NB = (uint32_t)a.max_bins;
+    a.view0 = make_int4(k.gx, k.gy, 0, 0);
+    a.means2D = reinterpret_cast<const float2*>(pre->means2D);  // in index order: no order array
+    a.radii = pre->radii;
+    bin_layout(a);
+    G3_ARG(a.table2_len < 0xFFFFFFFFull, "binning table too large");
+    // Gaussian-sized scratch: the binning's tables, the tiles' rays, the long lists' counts, offsets and scan
+    const size_t np = scan_partials_needed((uint32_t)num_tiles + 1) + 1;
     void* ws2;
-    if ((st = gs_ws2_get(c, alg(un * 4) + alg(un * 8) + 2 * alg(L * 4) + alg(np * 8) + alg((size_t)num_tiles * 16) +
+    if ((st = gs_ws2_get(c, alg(bin_workspace_bytes(a)) + alg(np * 8) + alg((size_t)num_tiles * 16) +
                                 2 * alg(((size_t)num_tiles + 1) * 4) + alg(un * 64),
                          &ws2)))
         return st;
     char* w = static_cast<char*>(ws2);
-    uint32_t* order = reinterpret_cast<uint32_t*>(w); w += alg(un * 4);
-    uint2* rects = reinterpret_cast<uint2*>(w); w += alg(un * 8);
-    uint32_t* table = reinterpret_cast<uint32_t*>(w); w += alg(L * 4);
-    uint32_t* scanned = reinterpret_cast<uint32_t*>(w); w += alg(L * 4);
+    bin_carve(a, w); w += alg(bin_workspace_bytes(a));
     unsigned long long* partial = reinterpret_cast<unsigned long long*>(w); w += alg(np * 8);
     float4* rays = reinterpret_cast<float4*>(w); w += alg((size_t)num_tiles * 16);
     uint32_t* bigcnt = reinterpret_cast<uint32_t*>(w); w += alg(((size_t)num_tiles + 1) * 4);
@@ -1080,44 +1077,17 @@ extern "C" int gs_bin_tiles_3d(gs_ctx* c, int n, const gs_preprocessed* pre, con
         gs3::tile_rays_kernel<<<(num_tiles + 255) / 256, 256, 0, c->stream>>>(k, rays);
         G3_HIP(hipGetLastError(), "tile rays kernel");
     }
-    gs3::iota_kernel<<<(n + 255) / 256, 256, 0, c->stream>>>((uint32_t)n, order);
-    G3_HIP(hipGetLastError(), "iota kernel");
-    gsb::BinArgs a{};
-    a.V = 1;
-    a.N = n;
-    a.C = C;
-    a.G = G;
-    a.S = 0;
-    a.G1 = G;
-    a.sidx = order;
-    a.sidx_stride = 1;
-    a.means2D = reinterpret_cast<const float2*>(pre->means2D);
-    a.radii = pre->radii;
-    a.views = nullptr;
-    a.view0 = make_int4(k.gx, k.gy, 0, 0);
-    a.vblock0 = nullptr;
-    a.table = table;
-    a.table_len = L;
-    a.rects = rects;
-    a.out = values;
-    a.capacity = capacity;
-    a.overflow = ovf;
-    a.diff_len = (k.gx + 1) * (k.gy + 1);
-    const int blocks = bin_blocks(C, k.gx, k.gy, c->bin_tpl);
-    G3_HIP(launch_bin_count(a, blocks, c->bin_tpl, c->stream), "binning count kernel");
-    G3_HIP(launch_scan_u32_exclusive(table, (uint32_t)L, scanned, partial, c->stream, nullptr, total64),
-           "binning scan");
-    a.table = scanned;
     unsigned long long K = 0;
-    G3_HIP(hipMemcpyAsync(&K, total64, 8, hipMemcpyDeviceToHost, c->stream), "hipMemcpyAsync(total)");
-    G3_HIP(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+    if ((st = gs_bin_count(c, a, &K))) return st;
     if (total) *total = (long long)K;
     if (K > capacity)
         return gs_set_error(GS_ERR_CAPACITY, "gs_bin_tiles_3d: %llu pairs exceed capacity %u", K, capacity);
-    G3_HIP(launch_bin_ranges(a, scanned, (uint32_t)num_tiles, ranges, c->stream), "binning ranges kernel");
+    a.out = values;
+    a.capacity = capacity;
+    G3_HIP(launch_bin_ranges(a, ranges, c->stream), "binning ranges kernel");
     if (K == 0) return GS_OK;
     G3_ARG(values != nullptr, "null values buffer");
-    G3_HIP(launch_bin_place(a, blocks, c->bin_tpl, c->stream), "binning place kernel");
+    G3_HIP(launch_bin_place(a, c->stream), "binning place kernel");
     const float4* rays_arg = k.have_ivp ? rays : nullptr;
     gs3::pack_keys3d_kernel<<<(n + 255) / 256, 256, 0, c->stream>>>(n, pre->depths, pre3d->cov3D_inv,
                                                                      pre3d->mean_offset, packed);

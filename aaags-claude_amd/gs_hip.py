@@ -162,13 +162,13 @@ class GsHip:
         self._check(self.lib.gs_ctx_apply_tuning(self.ctx, ctypes.byref(t)), "gs_ctx_apply_tuning")
 
     def set_split(self, groups):
-        """Trainer forward: depth groups placed before the first raster round (0: one round)."""
+        """Stored with the tuning; no effect (the forward runs in one round)."""
         d = self.tuning()
         d["split_groups"] = int(groups)
         self.apply_tuning(d)
 
     def set_binning(self, group=0, tiles_per_lane=0):
-        """Direct-placement binning knobs (0 keeps the current value)."""
+        """Stored with the tuning (0 keeps the current value); no effect, the binning's layout follows the sizes."""
         self._check(self.lib.gs_ctx_set_binning(self.ctx, _i32(group), _i32(tiles_per_lane)), "gs_ctx_set_binning")
 
     def sync(self):

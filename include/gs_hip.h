@@ -207,9 +207,10 @@ int gs_bin_sorted_words(gs_ctx* ctx, int n, const gs_preprocessed* pre, int widt
  * Sorter::sort (tile_binner.h:7-12, sorter.h:7; tile_binner_cpu.cpp:59-99,
  * sorter_cpu.cpp:6-44).  values[0..K) and ranges are exactly the values_out
  * and ranges of gs_sort_pairs on the duplicate-with-keys pairs; the keys are
- * not produced.  The Gaussians are stably sorted by depth bits, then each
- * index is written once, straight to its slot: per-tile counts over groups of
- * depth-ordered Gaussians, scanned tile-major, give every pair's position.
+ * not produced.  The Gaussians are stably sorted by depth bits and listed per
+ * bin of 4 x 4 or 8 x 8 tiles, then each index is written once, straight to
+ * its slot: per-tile counts over groups of a bin's list, scanned tile-major,
+ * give every pair's position.
  * K is read back and must not exceed `capacity`; `values` must be 16-byte
  * aligned.  Up to 255 x 255 tiles (GS_ERR_UNSUPPORTED beyond). */
 int gs_bin_tiles(gs_ctx* ctx, int n, const gs_preprocessed* pre, int width, int height, uint32_t* values,
@@ -485,14 +486,12 @@ typedef struct gs_tuning {
     int radix_bits;         /* depth-sort digit width: 4..8 */
     int raster_batch;       /* forward LDS batch depth: 64, 128, 256, 512 */
     int raster_bwd_batch;   /* backward LDS batch depth: 64, 128, 256 */
-    int bin_group;          /* Gaussians per binning group: power of two, 256..65536 */
-    int bin_tiles_per_lane; /* binning bin shape: 1, 2 or 4 (bin = 8 x 8*tpl tiles) */
+    int bin_group;          /* power of two, 256..65536; no effect (the binning's layout follows the sizes) */
+    int bin_tiles_per_lane; /* 1, 2 or 4; no effect */
     int persistent_per_cu;  /* batched raster: persistent groups per CU (0: one group per tile) */
     float binning_ms, raster_fwd_ms, raster_bwd_ms; /* best times measured */
-    int split_groups;       /* single-view forward: groups of 1024 nearest Gaussians placed before the
-                             * first raster round; the rest is placed only for bins with unfinished
-                             * tiles (0: one round) */
-    float forward_ms;       /* best forward (preprocess, binning, raster) measured with that split */
+    int split_groups;       /* >= 0; no effect (the forward runs in one round) */
+    float forward_ms;       /* the whole forward (preprocess, binning, raster) with the knobs chosen */
 } gs_tuning;
 
 /* Current knobs of a context (times zero) / set all knobs at once (for a

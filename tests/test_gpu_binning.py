@@ -1,0 +1,92 @@
+"""The two-level binning (gs_bin_tiles and its users) at the sizes where its
+layout changes: one bin, one chunk and one more Gaussian, the largest view
+with 4 x 4-tile bins and the next one, Gaussians over more bins than a lane
+handles alone, and record buffers that the first guess does not fill."""
+import numpy as np
+import pytest
+import torch
+
+from oracle.oracle import _rects
+from gs_scenes import RenderCfg, make_camera, random_small_scene, target_image
+from helpers import assert_image_close
+
+pytestmark = pytest.mark.gpu
+
+
+def _pre(n, width, height, max_radius, seed):
+    rng = np.random.default_rng(seed)
+    pre = dict(means2D=rng.uniform(0, 1, (n, 2)) * (width + 40, height + 40) - 20,
+               depths=rng.choice([0.5, 1.0, 2.0], n) + rng.integers(0, max(n // 4, 1), n) / max(n, 1),
+               conics=np.ones((n, 3)), op2d=np.ones(n), rgb=np.ones((n, 3)))
+    pre = {k: np.ascontiguousarray(v, np.float32) for k, v in pre.items()}
+    r = np.exp(rng.uniform(0, np.log(max_radius), n)).astype(np.int32)
+    r[rng.random(n) < 0.1] = 0  # culled
+    pre["radii"] = r
+    x0, y0, x1, y1 = _rects(pre["means2D"], r, width, height)
+    pre["tiles"] = ((x1 - x0) * (y1 - y0) * (r > 0)).astype(np.int32)
+    return pre
+
+
+@pytest.mark.parametrize("n,width,height,max_radius", [
+    (1, 16, 16, 30), (255, 64, 64, 40), (256, 65, 64, 40), (257, 80, 130, 100), (5000, 411, 307, 60),
+    (140_000, 500, 400, 12),            # chunks of 512 Gaussians
+    (3000, 2048, 2048, 300),            # 1024 bins of 4 x 4 tiles
+    (3000, 2064, 2048, 300),            # bins of 8 x 8 tiles
+    (500, 4080, 4080, 900),             # the largest view: 255 x 255 tiles
+    (400, 1920, 1080, 4000),            # most Gaussians cover the view: the record buffer grows
+])
+def test_binning_equals_sorted_pairs(oracle, n, width, height, max_radius):
+    from gs_hip import GsHip
+    print("[case] binning", n, width, height, max_radius, flush=True)
+    hip = GsHip(0)  # own context: its buffers start empty
+    pre = _pre(n, width, height, max_radius, n + width)
+    tiles = ((width + 15) // 16) * ((height + 15) // 16)
+    keys, vals = oracle.duplicate(pre, n, width, height)
+    ks, vs, ranges = oracle.sort_pairs(keys, vals, tiles)
+    dev = {k: torch.tensor(v, device=hip.dev) for k, v in pre.items()}
+    for _ in range(2):  # the second call finds the buffers grown
+        got, rg, K = hip.bin_tiles(dev, width, height)
+        assert K == len(vs)
+        assert np.array_equal(got.cpu().numpy().view(np.uint32), vs)
+        assert np.array_equal(rg.cpu().numpy().view(np.uint32), np.asarray(ranges).reshape(-1))
+    assert not hip.check_overflow()
+
+
+def _wide_scene():
+    scene, _, _ = random_small_scene(600, 1, 17, logscale=(-0.6, 0.2), op=(-4.0, 0.5))
+    return scene, make_camera((0.0, 0.0, -3.0), 1920, 1072, 60.0)
+
+
+def test_trainer_redoes_when_records_outgrow_buffer(oracle):
+    """A frame whose bin records outgrow the buffer that an earlier small view
+    left (its pair count is then cut short too) is redone with larger ones."""
+    from gs_hip import GsHip, GsTrainer
+    print("[case] trainer record overflow", flush=True)
+    hip = GsHip(0)
+    scene, near = _wide_scene()
+    far = make_camera((0.0, 0.0, -12.0), 64, 48, 60.0)
+    cfg = RenderCfg(sh_degree=1, training=True)
+    tr = GsTrainer(hip, scene)
+    tr.render(far, cfg)
+    K = tr.render(near, cfg)
+    ref = oracle.forward(scene, near, cfg)
+    assert K == len(ref["keys"])
+    assert_image_close(tr.buffer("image", (near.height, near.width, 3)).cpu().numpy(), ref["img"])
+    assert not hip.check_overflow()
+
+
+def test_batch_grows_record_buffer(oracle):
+    from gs_hip import GsBatch, GsHip, GsTrainer
+    print("[case] batch record overflow", flush=True)
+    hip = GsHip(0)
+    scene, near = _wide_scene()
+    small = make_camera((0.0, 0.0, -6.0), 50, 37, 60.0)
+    cfg = RenderCfg(sh_degree=1, training=True)
+    tr = GsTrainer(hip, scene)
+    cams = [small, near]
+    b = GsBatch(tr, cams, cfg, [target_image(c.width, c.height, 4) for c in cams])
+    K = b.render()
+    refs = [oracle.forward(scene, c, cfg) for c in cams]
+    assert K == sum(len(r["keys"]) for r in refs)
+    for img, r in zip(b.images(), refs):
+        assert_image_close(img.cpu().numpy(), r["img"])
