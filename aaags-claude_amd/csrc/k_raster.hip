@@ -14,7 +14,9 @@
 // nine per-Gaussian gradient terms are summed across the wave with packed
 // permlane-swap/DPP steps (no LDS traffic), across the four waves with LDS
 // atomics, and land in HBM with one float atomic per (tile, Gaussian,
-// component).
+// component), issued by consecutive lanes per Gaussian.  What bounds the
+// backward: VALU issue (71 instructions per visited entry and wave, 27 of them
+// the sums), and below about two workgroups per CU the latency of that chain.
 //
 // Multi-view: the same tile bodies run over a global (view, tile) list, either
 // one workgroup per global tile or a persistent grid that takes tiles from
@@ -235,14 +237,11 @@ __device__ __forceinline__ void fwd_tile(const RasterArgs& a, int tile, FwdSmem<
     }
 }
 
-// ---- packed wave reduction of the nine gradient terms ----------------------
-// Summing nine values over 64 lanes one by one costs 9 x 6 cross-lane steps.
+// ---- packed wave reduction of the gradient terms ---------------------------
 // Packed, two values share each exchange: v_permlane32_swap leaves value a
 // summed over lane pairs {l, l+32} in lanes 0-31 and value b in lanes 32-63;
-// v_permlane16_swap does the same between 16-lane rows; DPP row rotations
-// finish each row.  Afterwards row r (lanes 16r..16r+15) holds, in every lane,
-//   k0 = term A[r], k1 = term 4 + A[r], with A = {0, 2, 1, 3},
-// and k2 = term 8 everywhere.
+// v_permlane16_swap does the same between 16-lane rows.  swap16_sum of
+// swap32_sum(a, b) and swap32_sum(c, d) holds a, c, b, d in rows 0 .. 3.
 __device__ __forceinline__ float swap32_sum(float a, float b) {
     auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
@@ -258,50 +257,61 @@ __device__ __forceinline__ float dpp_f(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
 }
 
-// Sum over the 16 lanes of each row (row_ror:8, 4, 2, 1).
-__device__ __forceinline__ float row_sum(float v) {
-    v += dpp_f<0x128>(v);
-    v += dpp_f<0x124>(v);
-    v += dpp_f<0x122>(v);
-    v += dpp_f<0x121>(v);
-    return v;
-}
-
-// Which reduced sum a lane delivers: in row r (lanes 16r .. 16r+15), lane
-// 16r delivers k0 (term A[r]) and lane 16r+1 k1 (term 4 + A[r]); lane 2
-// delivers k2 (term 8).  Fixed per lane, so it is set up once per thread and
-// the delivery below is selects, not branches.
+// The nine sums of one visited entry over a wave's strip of 16 columns x 4
+// rows (lane l at column l % 16, row l / 16).  dx depends on the column alone
+// and dy on the row alone, so the six sums of dop times 1, dx, dy, dx^2, dx dy,
+// dy^2 start as three values (dop, dop dy, dop dy^2) summed over the rows, and
+// are multiplied by dx afterwards:
+//   swap steps (rows): k0 = {dop, dop dy^2, dop dy, c0} and k1 = {c1, c1, c2,
+//     c2} in rows 0 .. 3, each summed over the four rows, per column;
+//   m1 = k0 dx and m2 = m1 dx carry the dx and dx^2 sums; row 1 and 3 of m1
+//     hold nothing wanted, so k1 goes there;
+//   DPP steps (columns): the values share a register as soon as their sums
+//     repeat within a row: m1 takes the upper half of each row after the first
+//     step, m2 the odd quarters after the second.
+// 22 VALU instructions after the four products; nine separate terms took 28
+// after eight products, and two selects to deliver (200k Gaussians at 720p:
+// 343 -> 332 us, 10k at 256 x 256: 82 -> 77 us).
 struct ReduceRole {
-    bool is0, is1, any;
-    int term;
+    bool odd_row, half, quarter;  // lane / 16 odd; lane & 8; lane & 4
+    int term;                     // the sum this lane delivers (-1: none)
 };
 
 __device__ __forceinline__ ReduceRole reduce_role(int lane) {
-    const int r = lane >> 4, p = lane & 15;
-    const int a = ((r & 1) << 1) | (r >> 1);
     ReduceRole q;
-    q.is0 = p == 0;
-    q.is1 = p == 1;
-    q.any = q.is0 || q.is1 || lane == 2;
-    q.term = q.is0 ? a : (q.is1 ? 4 + a : 8);
+    const int row = lane >> 4, p = lane & 15;
+    q.odd_row = (row & 1) != 0;
+    q.half = (lane & 8) != 0;
+    q.quarter = (lane & 4) != 0;
+    q.term = -1;
+    if (p == 0) q.term = row == 0 ? 8 : (row == 1 ? 4 : (row == 2 ? 1 : 5));  // k0: 1, dy^2, dy, c0
+    if (p == 8) q.term = row == 0 ? 0 : (row == 1 ? 6 : (row == 2 ? 3 : 7));  // m1: dx, c1, dx dy, c2
+    if (p == 4 && row == 0) q.term = 2;                                       // m2: dx^2
     return q;
 }
 
-// Reduces gv[0..8] over the wave; the nine lanes with q.any set return one
-// distinct term's sum each (term q.term).
-__device__ __forceinline__ float wave_reduce9(const float (&gv)[NG], const ReduceRole& q) {
-    const float h0 = swap32_sum(gv[0], gv[1]);
-    const float h1 = swap32_sum(gv[2], gv[3]);
-    const float h2 = swap32_sum(gv[4], gv[5]);
-    const float h3 = swap32_sum(gv[6], gv[7]);
-    const float h4 = swap32_sum(gv[8], gv[8]);
+__device__ __forceinline__ float wave_reduce9(float dop, float dx, float dy, float c0, float c1, float c2,
+                                              const ReduceRole& q) {
+    const float py = dop * dy;
+    const float h0 = swap32_sum(dop, py);
+    const float h1 = swap32_sum(py * dy, c0);
+    const float h2 = swap32_sum(c1, c2);
     float k0 = swap16_sum(h0, h1);
-    float k1 = swap16_sum(h2, h3);
-    float k2 = swap16_sum(h4, h4);
-    k0 = row_sum(k0);
-    k1 = row_sum(k1);
-    k2 = row_sum(k2);
-    return q.is0 ? k0 : (q.is1 ? k1 : k2);
+    const float k1 = swap16_sum(h2, h2);
+    float m1 = k0 * dx;
+    float m2 = m1 * dx;
+    m1 = q.odd_row ? k1 : m1;
+    constexpr int ROR8 = 0x128, HALF_MIRROR = 0x141, QUAD_XOR2 = 0x4E, QUAD_XOR1 = 0xB1;
+    k0 += dpp_f<ROR8>(k0);
+    m1 += dpp_f<ROR8>(m1);
+    m2 += dpp_f<ROR8>(m2);
+    k0 = q.half ? m1 : k0;
+    k0 += dpp_f<HALF_MIRROR>(k0);
+    m2 += dpp_f<HALF_MIRROR>(m2);
+    k0 = q.quarter ? m2 : k0;
+    k0 += dpp_f<QUAD_XOR2>(k0);
+    k0 += dpp_f<QUAD_XOR1>(k0);
+    return k0;
 }
 
 struct PixIn {
@@ -410,17 +420,6 @@ __device__ __forceinline__ void bwd_tile(const RasterArgs& a, int tile, BwdSmem<
                 // leave LDS (alpha >= 0.99 is the clamp: no gradient)
                 const float dop = (contrib && alpha < 0.99f) ? dal * ep : 0.0f;
                 const float aT = contrib ? alpha * Ti : 0.0f;
-                const float pdx = dop * dx, pdy = dop * dy;
-                float gv[NG];
-                gv[0] = pdx;
-                gv[1] = pdy;
-                gv[2] = pdx * dx;
-                gv[3] = pdx * dy;
-                gv[4] = pdy * dy;
-                gv[5] = aT * dC0;
-                gv[6] = aT * dC1;
-                gv[7] = aT * dC2;
-                gv[8] = dop;
                 // colour behind the next entry: alpha c + (1 - alpha) acc
                 const float ac = contrib ? alpha : 0.0f;
                 {
@@ -431,32 +430,42 @@ __device__ __forceinline__ void bwd_tile(const RasterArgs& a, int tile, BwdSmem<
                 }
                 T = contrib ? Ti : T;
                 if (__ballot(contrib) != 0ull) {
-                    const float v = wave_reduce9(gv, role);
-                    if (role.any && v != 0.0f) atomicAdd(&sm.g[k][role.term], v);
+                    const float v = wave_reduce9(dop, dx, dy, aT * dC0, aT * dC1, aT * dC2, role);
+                    if (role.term >= 0 && v != 0.0f) atomicAdd(&sm.g[k][role.term], v);
                 }
             }
         }
         __syncthreads();
-        for (int k = t; k < n; k += 256) {
+        // One (Gaussian, term) per thread, nine consecutive lanes per Gaussian:
+        // its atomics into one array are one request per line, four or five for
+        // the nine terms.  With a thread per Gaussian and nine instructions of
+        // 64 scattered lines each, the atomics held the kernel up by 105 us at
+        // 1M Gaussians and 1080p (612 -> 474 us with this order), 332 -> 263 us
+        // at 200k and 720p.
+        // Sums of dop * (dx, dy, dx^2, dx dy, dy^2); times the opacity they are
+        // those of dpow, and -> the reference's terms
+        // (rasterizer_backward_cpu.cpp): d_mean = -(a Sx + b Sy, c Sy + b Sx),
+        // d_conic = (-Sxx / 2, -Sxy, -Syy / 2); the staged conic is
+        // (-a/2, -b, -c/2, o)
+        for (int i = t; i < n * NG; i += 256) {
+            const int k = i / NG, c = i - k * NG;
             const uint32_t id = sm.id[k];
-            // sums of dop * (dx, dy, dx^2, dx*dy, dy^2); times the opacity
-            // they are those of dpow, and -> the reference's terms
-            // (rasterizer_backward_cpu.cpp): d_mean = -(a Sx + b Sy, c Sy + b Sx),
-            // d_conic = (-Sxx / 2, -Sxy, -Syy / 2); the staged conic is
-            // (-a/2, -b, -c/2, o)
-            const float4 cs = sm.e[k].co;
-            const float ca = -2.0f * cs.x, cb = -cs.y, cc = -2.0f * cs.z, op = cs.w;
-            const float sx = op * sm.g[k][0], sy = op * sm.g[k][1];
-            float v;
-            v = -(ca * sx + cb * sy); if (v != 0.0f) unsafeAtomicAdd(&g.d_means2D[id].x, v);
-            v = -(cc * sy + cb * sx); if (v != 0.0f) unsafeAtomicAdd(&g.d_means2D[id].y, v);
-            v = -0.5f * (op * sm.g[k][2]); if (v != 0.0f) unsafeAtomicAdd(&g.d_conics[id * 3 + 0], v);
-            v = -(op * sm.g[k][3]); if (v != 0.0f) unsafeAtomicAdd(&g.d_conics[id * 3 + 1], v);
-            v = -0.5f * (op * sm.g[k][4]); if (v != 0.0f) unsafeAtomicAdd(&g.d_conics[id * 3 + 2], v);
-            v = sm.g[k][5]; if (v != 0.0f) unsafeAtomicAdd(&g.d_rgb[id * 3 + 0], v);
-            v = sm.g[k][6]; if (v != 0.0f) unsafeAtomicAdd(&g.d_rgb[id * 3 + 1], v);
-            v = sm.g[k][7]; if (v != 0.0f) unsafeAtomicAdd(&g.d_rgb[id * 3 + 2], v);
-            v = sm.g[k][8]; if (v != 0.0f) unsafeAtomicAdd(&g.d_op[id], v);
+            float v = (&sm.g[0][0])[i];
+            float* dst;
+            if (c < 5) {
+                const float4 cs = sm.e[k].co;
+                if (c < 2) {
+                    const float ca = -2.0f * (c == 0 ? cs.x : cs.z), cb = -cs.y;
+                    v = -(ca * (cs.w * v) + cb * (cs.w * sm.g[k][1 - c]));
+                    dst = &g.d_means2D[id].x + c;
+                } else {
+                    v = (c == 3 ? -1.0f : -0.5f) * (cs.w * v);
+                    dst = g.d_conics + (size_t)id * 3 + (c - 2);
+                }
+            } else {
+                dst = c < 8 ? g.d_rgb + (size_t)id * 3 + (c - 5) : g.d_op + id;
+            }
+            if (v != 0.0f) unsafeAtomicAdd(dst, v);
         }
         hi = lo;
     }
