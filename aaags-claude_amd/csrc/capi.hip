@@ -629,23 +629,40 @@ int gs_bin_finish(gs_ctx* c, uint32_t* values, uint32_t capacity, uint32_t* rang
     return GS_OK;
 }
 
+extern "C" int gs_bin_tiles_count(gs_ctx* c, int n, const gs_preprocessed* pre, int width, int height,
+                                  long long* total) {
+    GS_CHECK_ARG(c != nullptr && total != nullptr, "null argument");
+    int st = gs_bin_prepare(c, n, pre, width, height, total, nullptr, nullptr);
+    if (st) return st;
+    c->bin_pairs = *total;
+    return GS_OK;
+}
+
+extern "C" int gs_bin_tiles_place(gs_ctx* c, uint32_t* values, uint32_t capacity, uint32_t* ranges) {
+    GS_CHECK_ARG(c != nullptr, "null context");
+    GS_CHECK_ARG(c->bin_pending, "gs_bin_tiles_place: no prepared binning on this context");
+    GS_CHECK_ARG(ranges != nullptr, "null tile ranges");
+    GS_CHECK_ARG(aligned(values, 16) || values == nullptr, "values must be 16-byte aligned");
+    if (c->bin_pairs > (long long)capacity) {
+        c->bin_pending = false;
+        return gs_set_error(GS_ERR_CAPACITY, "gs_bin_tiles: %lld pairs exceed capacity %u", c->bin_pairs, capacity);
+    }
+    if (c->bin_pairs > 0 && !values) {
+        c->bin_pending = false;
+        return gs_set_error(GS_ERR_INVALID, "null values buffer");
+    }
+    return gs_bin_finish(c, values, capacity, ranges);
+}
+
 extern "C" int gs_bin_tiles(gs_ctx* c, int n, const gs_preprocessed* pre, int width, int height, uint32_t* values,
                             uint32_t capacity, uint32_t* ranges, long long* total_host) {
     GS_CHECK_ARG(ranges != nullptr, "null tile ranges");
     GS_CHECK_ARG(aligned(values, 16) || values == nullptr, "values must be 16-byte aligned");
     long long K = 0;
-    int st = gs_bin_prepare(c, n, pre, width, height, &K, nullptr, nullptr);
+    int st = gs_bin_tiles_count(c, n, pre, width, height, &K);
     if (st) return st;
     if (total_host) *total_host = K;
-    if (K > (long long)capacity) {
-        c->bin_pending = false;
-        return gs_set_error(GS_ERR_CAPACITY, "gs_bin_tiles: %lld pairs exceed capacity %u", K, capacity);
-    }
-    if (K > 0 && !values) {
-        c->bin_pending = false;
-        return gs_set_error(GS_ERR_INVALID, "null values buffer");
-    }
-    return gs_bin_finish(c, values, capacity, ranges);
+    return gs_bin_tiles_place(c, values, capacity, ranges);
 }
 
 static gsr::RasterArgs raster_args(int width, int height, const gs_preprocessed* pre, const uint32_t* values,

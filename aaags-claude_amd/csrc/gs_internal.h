@@ -39,8 +39,9 @@ struct gs_ctx {
     int split_groups = 64;      // likewise: the forward no longer runs in two rounds
     void* coarse = nullptr;     // the binning's bin records
     size_t coarse_bytes = 0;
-    gsb::BinArgs* bin = nullptr;  // the binning that gs_bin_begin left for gs_bin_place
+    gsb::BinArgs* bin = nullptr;  // the binning that gs_bin_prepare left for gs_bin_finish
     bool bin_pending = false;
+    long long bin_pairs = 0;      // its pair count, once read back
 };
 
 int gs_set_error(int code, const char* fmt, ...);

@@ -99,6 +99,8 @@ def load_library(path: str = LIB_PATH):
         _LIB.gs_scan_tiles.argtypes = [_vp, _i32, _vp, _vp, _vp, _vp]
         _LIB.gs_bin_sorted_words.argtypes = [_vp, _i32, _vp, _i32, _i32, _vp, _u32, _vp, _vp]
         _LIB.gs_bin_tiles.argtypes = [_vp, _i32, _vp, _i32, _i32, _vp, _u32, _vp, _vp]
+        _LIB.gs_bin_tiles_count.argtypes = [_vp, _i32, _vp, _i32, _i32, _vp]
+        _LIB.gs_bin_tiles_place.argtypes = [_vp, _vp, _u32, _vp]
         _LIB.gs_ctx_set_binning.argtypes = [_vp, _i32, _i32]
     return _LIB
 
@@ -293,12 +295,13 @@ class GsHip:
         num_tiles = ((width + 15) // 16) * ((height + 15) // 16)
         ranges = torch.empty(num_tiles * 2, dtype=torch.int32, device=self.dev)
         K = ctypes.c_longlong()
-        if capacity is None:
-            st = self.lib.gs_bin_tiles(self.ctx, n, ctypes.byref(self._pre_struct(pre)), width, height, None, _u32(0),
-                                       _vp(ptr(ranges)), ctypes.byref(K))
-            if st not in (0, 3):
-                self._check(st, "gs_bin_tiles")
-            capacity = max(int(K.value), 1)
+        if capacity is None:  # counted first, then allocated and placed
+            self._check(self.lib.gs_bin_tiles_count(self.ctx, n, ctypes.byref(self._pre_struct(pre)), width, height,
+                                                    ctypes.byref(K)), "gs_bin_tiles_count")
+            values = torch.empty(max(int(K.value), 1), dtype=torch.int32, device=self.dev)
+            self._check(self.lib.gs_bin_tiles_place(self.ctx, ptr(values), values.numel(), ptr(ranges)),
+                        "gs_bin_tiles_place")
+            return values[:K.value], ranges, int(K.value)
         values = torch.empty(capacity, dtype=torch.int32, device=self.dev)
         self._check(self.lib.gs_bin_tiles(self.ctx, n, ctypes.byref(self._pre_struct(pre)), width, height,
                                           _vp(ptr(values)), _u32(capacity), _vp(ptr(ranges)), ctypes.byref(K)),
@@ -505,15 +508,15 @@ class GsHip:
     def l1_loss(self, img, gt):
         H, W = img.shape[0], img.shape[1]
         d_img = torch.empty_like(img)
-        loss = torch.zeros(1, dtype=torch.float64, device=self.dev)
+        loss = torch.empty(1, dtype=torch.float64, device=self.dev)
         self._check(self.lib.gs_l1_loss(self.ctx, W, H, _vp(ptr(img)), _vp(ptr(gt)), _vp(ptr(d_img)), _vp(ptr(loss))),
                     "gs_l1_loss")
         return loss, d_img
 
     def alloc_rgrads(self, n):
-        d = self.dev
-        return dict(d_means2D=torch.zeros((n, 2), device=d), d_conics=torch.zeros((n, 3), device=d),
-                    d_rgb=torch.zeros((n, 3), device=d), d_op2d=torch.zeros(n, device=d))
+        block = torch.zeros(9 * n, device=self.dev)  # one fill
+        return dict(d_means2D=block[:2 * n].view(n, 2), d_conics=block[2 * n:5 * n].view(n, 3),
+                    d_rgb=block[5 * n:8 * n].view(n, 3), d_op2d=block[8 * n:])
 
     def raster_bwd(self, pre, values_sorted, ranges, width, height, px, d_image, bg=(0.0, 0.0, 0.0), rg=None):
         n = pre["radii"].numel() if "radii" in pre else pre["op2d"].numel()
@@ -534,7 +537,12 @@ class GsHip:
                     rot=torch.zeros((n, 4), device=d), sh=torch.zeros((n, k, 3), device=d), op=torch.zeros(n, device=d))
 
     def preprocess_bwd(self, p, cam, cfg, radii, rg, out=None, accumulate=False):
-        out = out if out is not None else self.alloc_pgrads(p["n"], p["max_coeffs"])
+        if out is None:
+            n, k, d = p["n"], p["max_coeffs"], self.dev
+            # without accumulate every entry is written
+            out = self.alloc_pgrads(n, k) if accumulate else dict(
+                pos=torch.empty((n, 3), device=d), scale=torch.empty((n, 3), device=d),
+                rot=torch.empty((n, 4), device=d), sh=torch.empty((n, k, 3), device=d), op=torch.empty(n, device=d))
         g = self._gauss(p, raw=True)
         c, f = cam.to_c(), cfg.to_c()
         rgs = _RGrads(ptr(rg["d_means2D"]), ptr(rg["d_conics"]), ptr(rg["d_rgb"]), ptr(rg["d_op2d"]))

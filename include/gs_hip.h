@@ -215,6 +215,15 @@ int gs_bin_sorted_words(gs_ctx* ctx, int n, const gs_preprocessed* pre, int widt
  * aligned.  Up to 255 x 255 tiles (GS_ERR_UNSUPPORTED beyond). */
 int gs_bin_tiles(gs_ctx* ctx, int n, const gs_preprocessed* pre, int width, int height, uint32_t* values,
                  uint32_t capacity, uint32_t* ranges, long long* total_host);
+/* gs_bin_tiles in two calls, for callers that allocate `values` once they know
+ * the pair count: the first does everything up to the count (read back into
+ * *total), the second places the pairs and writes the ranges.  The prepared
+ * lists live in the context's workspace: the next call on the context must be
+ * the second one (any other binning or sorting call drops them, and the second
+ * call then fails with GS_ERR_INVALID).  A capacity below the count is refused
+ * (GS_ERR_CAPACITY), as by gs_bin_tiles. */
+int gs_bin_tiles_count(gs_ctx* ctx, int n, const gs_preprocessed* pre, int width, int height, long long* total);
+int gs_bin_tiles_place(gs_ctx* ctx, uint32_t* values, uint32_t capacity, uint32_t* ranges);
 
 /* Forward rasterization: Rasterizer::rasterize (rasterizer.h:7-15), the
  * rasterize kernel (gpu/kernels/rasterize.cl:10-274, 2D lines) and

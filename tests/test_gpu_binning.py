@@ -90,3 +90,19 @@ def test_batch_grows_record_buffer(oracle):
     assert K == sum(len(r["keys"]) for r in refs)
     for img, r in zip(b.images(), refs):
         assert_image_close(img.cpu().numpy(), r["img"])
+
+
+def test_counted_binning_is_dropped_by_other_work(oracle):
+    """gs_bin_tiles_place after another binning call on the context fails instead of placing its lists."""
+    import ctypes
+    from gs_hip import GsHip
+    hip = GsHip(0)
+    pre = _pre(300, 200, 100, 30, 9)
+    dev = {k: torch.tensor(v, device=hip.dev) for k, v in pre.items()}
+    K = ctypes.c_longlong()
+    ps = hip._pre_struct(dev)
+    hip._check(hip.lib.gs_bin_tiles_count(hip.ctx, 300, ctypes.byref(ps), 200, 100, ctypes.byref(K)), "count")
+    hip.bin_sorted_words(dev, 200, 100)
+    values = torch.empty(max(K.value, 1), dtype=torch.int32, device=hip.dev)
+    ranges = torch.empty(2 * 13 * 7, dtype=torch.int32, device=hip.dev)
+    assert hip.lib.gs_bin_tiles_place(hip.ctx, values.data_ptr(), values.numel(), ranges.data_ptr()) == 1
