@@ -2,8 +2,8 @@
 //
 // scan:       reduce-then-scan over 4096-element blocks (three launches); the
 //             wave-level prefix uses lane shuffles, the block level LDS.
-// duplicate:  one thread per Gaussian writes its tile|depth keys at the
-//             scanned offset (row-major over its tile rectangle).
+// duplicate:  a wave writes the tile|depth keys of 64 Gaussians at their
+//             scanned offsets (row-major over each tile rectangle).
 // radix sort: per pass an upsweep (per-block digit histogram), a scan of each
 //             digit's row of the digit-major histogram table (one wave per
 //             digit), and a downsweep that adds the digit totals' scan, ranks keys
@@ -154,31 +154,67 @@ __global__ __launch_bounds__(SCAN_THREADS) void scan_downsweep_kernel(const TIn*
 
 // ----------------------------------------------------------- duplicate ----
 // tile_binner_cpu.cpp:59-99: keys tile_id << 32 | float bits of the depth.
+// A wave takes 64 Gaussians and deals their pairs out evenly: lane l writes
+// pairs l, l + 64, ... of the wave's concatenated rectangles, finding each
+// pair's Gaussian by a binary search of the 64 running counts in LDS.  The
+// Gaussians' pairs follow each other in the output too, so the stores are
+// whole runs, and no lane waits for the largest rectangle of its wave (one
+// lane per Gaussian, its pairs one by one: 115 us for the 200k Gaussians of a
+// 1280 x 720 view, now 15 us).
 __global__ __launch_bounds__(256) void duplicate_kernel(int n, const float2* __restrict__ means2D,
                                                         const float* __restrict__ depths, const int* __restrict__ radii,
                                                         const uint32_t* __restrict__ offsets_incl, int gx, int gy,
                                                         uint64_t* __restrict__ keys, uint32_t* __restrict__ values,
                                                         uint32_t capacity, uint32_t* __restrict__ overflow) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    int r = radii[i];
-    if (r <= 0) return;
-    float2 m = means2D[i];
-    int mn[2], mx[2];
-    gsd::get_rect(m.x, m.y, r, gx, gy, mn, mx);
-    uint32_t cnt = (uint32_t)((mx[1] - mn[1]) * (mx[0] - mn[0]));
-    uint32_t off = offsets_incl[i] - cnt;
-    uint64_t db = (uint64_t)__float_as_uint(depths[i]);
-    for (int y = mn[1]; y < mx[1]; y++)
-        for (int x = mn[0]; x < mx[0]; x++) {
-            if (off < capacity) {
-                keys[off] = ((uint64_t)(uint32_t)(y * gx + x) << 32) | db;
-                values[off] = (uint32_t)i;
-            } else if (overflow) {
-                *overflow = 1u;
-            }
-            off++;
+    struct Item {
+        uint32_t first;  // output slot of pair 0
+        uint32_t tile0;  // its tile
+        uint32_t width;  // of the rectangle, in tiles
+        uint32_t depth;
+    };
+    __shared__ Item s_item[4][64];
+    __shared__ uint32_t s_end[4][64];  // running pair count of the wave
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int w = threadIdx.x >> 6, l = lane_id();
+    uint32_t cnt = 0u;
+    Item it{0u, 0u, 1u, 0u};
+    if (i < n) {
+        const int r = radii[i];
+        if (r > 0) {
+            const float2 m = means2D[i];
+            int mn[2], mx[2];
+            gsd::get_rect(m.x, m.y, r, gx, gy, mn, mx);
+            it.width = (uint32_t)(mx[0] - mn[0]);
+            cnt = (uint32_t)(mx[1] - mn[1]) * it.width;
+            it.first = offsets_incl[i] - cnt;
+            it.tile0 = (uint32_t)(mn[1] * gx + mn[0]);
+            it.depth = __float_as_uint(depths[i]);
         }
+    }
+    const uint32_t end = wave_inclusive_scan(cnt);
+    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)end, 63);
+    s_item[w][l] = it;
+    s_end[w][l] = end;
+    __syncthreads();
+    const uint32_t i0 = (uint32_t)(i - l);
+    bool dropped = false;
+    for (uint32_t p = (uint32_t)l; p < total; p += 64u) {
+        uint32_t j = 0u;  // the first Gaussian whose running count exceeds p
+#pragma unroll
+        for (uint32_t step = 32u; step > 0u; step >>= 1)
+            if (s_end[w][j + step - 1u] <= p) j += step;
+        const Item x = s_item[w][j];
+        const uint32_t k = p - (j > 0u ? s_end[w][j - 1u] : 0u);
+        const uint32_t y = k / x.width;
+        const uint32_t off = x.first + k;
+        if (off < capacity) {
+            keys[off] = ((uint64_t)(x.tile0 + y * (uint32_t)gx + (k - y * x.width)) << 32) | x.depth;
+            values[off] = i0 + j;
+        } else {
+            dropped = true;
+        }
+    }
+    if (dropped && overflow) *overflow = 1u;
 }
 
 // ------------------------------------------------- depth-ordered binning ----

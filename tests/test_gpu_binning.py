@@ -92,6 +92,30 @@ def test_batch_grows_record_buffer(oracle):
         assert_image_close(img.cpu().numpy(), r["img"])
 
 
+@pytest.mark.parametrize("n,width,height,max_radius", [(1, 16, 16, 5), (63, 300, 200, 80), (64, 300, 200, 80),
+                                                       (65, 300, 200, 600), (5000, 411, 307, 60), (300, 4200, 300, 900)])
+def test_duplicate_keys_equal_oracle(oracle, n, width, height, max_radius):
+    """Waves of one, 63, 64 and 65 Gaussians, empty rectangles among them, and
+    rectangles of the whole view; a capacity one short drops one pair and says so."""
+    from gs_hip import GsHip
+    print("[case] duplicate", n, width, height, flush=True)
+    hip = GsHip(0)
+    pre = _pre(n, width, height, max_radius, 3 * n + width)
+    if n == 1:
+        pre = dict(pre, radii=np.array([5], np.int32), means2D=np.array([[8.0, 8.0]], np.float32), tiles=np.array([1], np.int32))
+    keys, vals = oracle.duplicate(pre, n, width, height)
+    dev = {k: torch.tensor(v, device=hip.dev) for k, v in pre.items()}
+    offsets, K = hip.scan_tiles(dev["tiles"])
+    assert K == len(keys)
+    k, v = hip.duplicate(dev, offsets, K, width, height)
+    assert np.array_equal(k.cpu().numpy().view(np.uint64), keys)
+    assert np.array_equal(v.cpu().numpy().view(np.uint32), vals)
+    assert not hip.check_overflow()
+    k, v = hip.duplicate(dev, offsets, K, width, height, capacity=K - 1)
+    assert np.array_equal(k.cpu().numpy().view(np.uint64)[:K - 1], keys[:K - 1])
+    assert hip.check_overflow()
+
+
 def test_counted_binning_is_dropped_by_other_work(oracle):
     """gs_bin_tiles_place after another binning call on the context fails instead of placing its lists."""
     import ctypes
