@@ -153,7 +153,43 @@ struct PixOut {
     uint32_t* last_contrib;
 };
 
-template <int BATCH>
+// An entry at a pixel: the exponent and min(0.99, opacity e^power), with the
+// 1/255 decision exact (gsd::alpha_fast / alpha_fix); ep = e^power.
+struct Eval {
+    float dx, dy, power, ep, alpha;
+};
+
+__device__ __forceinline__ Eval evaluate(const Staged& e, float fpx, float fpy) {
+    Eval v;
+    const float2 mm = e.xy;
+    const float4 co = e.co;
+    v.dx = mm.x - fpx;
+    v.dy = mm.y - fpy;
+    v.power = power_of(co, v.dx, v.dy);
+    v.alpha = gsd::raster_alpha_wave(co.w, v.power, &v.ep);
+    return v;
+}
+
+// Two entries whose chains (LDS reads, power, exponential) overlap.
+__device__ __forceinline__ void evaluate2(const Staged& e0, const Staged& e1, float fpx, float fpy, Eval& a, Eval& b) {
+    const float2 m0 = e0.xy, m1 = e1.xy;
+    const float4 c0 = e0.co, c1 = e1.co;
+    a.dx = m0.x - fpx;
+    a.dy = m0.y - fpy;
+    b.dx = m1.x - fpx;
+    b.dy = m1.y - fpy;
+    a.power = power_of(c0, a.dx, a.dy);
+    b.power = power_of(c1, b.dx, b.dy);
+    bool n0, n1;
+    a.alpha = gsd::alpha_fast(c0.w, a.power, &a.ep, &n0);
+    b.alpha = gsd::alpha_fast(c1.w, b.power, &b.ep, &n1);
+    if (__ballot(n0 || n1) != 0ull) {
+        gsd::alpha_fix(c0.w, a.power, n0, &a.alpha, &a.ep);
+        gsd::alpha_fix(c1.w, b.power, n1, &b.alpha, &b.ep);
+    }
+}
+
+template <int BATCH, bool PAIR>
 __device__ __forceinline__ void fwd_tile(const RasterArgs& a, int tile, FwdSmem<BATCH>& sm, const PixOut& o) {
     const int tx = tile % a.gx, ty = tile / a.gx;
     const int t = threadIdx.x;
@@ -169,6 +205,32 @@ __device__ __forceinline__ void fwd_tile(const RasterArgs& a, int tile, FwdSmem<
     int cnt = 0;
     uint32_t last = 0;
     bool done = !inside;
+    // One visited entry, predicated: every lane runs it and selects, so the
+    // only branches are uniform (the CU's scalar unit, shared by its waves, is
+    // not spent on exec-mask bookkeeping of per-pixel branches).
+    auto blend = [&](const Eval& v, const float4& cl, uint32_t index, bool valid) {
+        // rasterizer_cpu.cpp: skip if power > 0 or alpha < 1/255; stop
+        // (without this entry) once T would fall below 1e-4
+        const bool use = valid && !done && v.power <= 0.0f && v.alpha >= 1.0f / 255.0f;
+        const float test_T = T * (1.0f - v.alpha);
+        const bool take = use && test_T >= 0.0001f;  // T and alpha are finite here
+        // used but no room left (one compare: the negated compare
+        // would be a second, since the compiler keeps NaN semantics)
+        done = done || (use != take);
+        // colour += c alpha T, with the weight alpha T selected in or out;
+        // the colour feeds no decision (T and alpha do), so its sums are
+        // contracted to FMAs
+        const float wt = take ? v.alpha * T : 0.0f;
+        {
+#pragma clang fp contract(fast)
+            C0 += cl.x * wt;
+            C1 += cl.y * wt;
+            C2 += cl.z * wt;
+        }
+        T = take ? test_T : T;
+        cnt += take ? 1 : 0;
+        last = take ? index : last;
+    };
     for (uint32_t base = start; base < end; base += BATCH) {
         if (__syncthreads_count(!done) == 0) break;
         for (int k = t; k < BATCH; k += 256) {
@@ -187,43 +249,27 @@ __device__ __forceinline__ void fwd_tile(const RasterArgs& a, int tile, FwdSmem<
         }
         __syncthreads();
         const int nc = (int)(((end - base) < (uint32_t)BATCH ? (end - base) : (uint32_t)BATCH) + 63u) >> 6;
-        // predicated: every lane runs every visited entry and selects, so the
-        // only branches are uniform (the CU's scalar unit, shared by its
-        // waves, is not spent on exec-mask bookkeeping of per-pixel branches)
         for (int c = 0; c < nc; c++) {
             if (__ballot(!done) == 0ull) break;
             uint64_t m = wave_uniform(sm.mask[w][c]);
             while (m != 0ull) {
-                const int k = (c << 6) + __builtin_ctzll(m);
-                m &= m - 1ull;
-                const float2 mm = sm.e[k].xy;
-                const float4 co = sm.e[k].co;
-                const float4 cl = sm.e[k].rgb;
-                const float dx = mm.x - fpx, dy = mm.y - fpy;
-                const float power = power_of(co, dx, dy);
-                float ep;
-                const float alpha = gsd::raster_alpha_wave(co.w, power, &ep);
-                // rasterizer_cpu.cpp: skip if power > 0 or alpha < 1/255; stop
-                // (without this entry) once T would fall below 1e-4
-                const bool use = !done && power <= 0.0f && alpha >= 1.0f / 255.0f;
-                const float test_T = T * (1.0f - alpha);
-                const bool take = use && test_T >= 0.0001f;  // T and alpha are finite here
-                // used but no room left (one compare: the negated compare
-                // would be a second, since the compiler keeps NaN semantics)
-                done = done || (use != take);
-                // colour += c alpha T, with the weight alpha T selected in or out;
-                // the colour feeds no decision (T and alpha do), so its sums are
-                // contracted to FMAs
-                const float wt = take ? alpha * T : 0.0f;
-                {
-#pragma clang fp contract(fast)
-                    C0 += cl.x * wt;
-                    C1 += cl.y * wt;
-                    C2 += cl.z * wt;
+                if constexpr (!PAIR) {
+                    const int k = (c << 6) + __builtin_ctzll(m);
+                    m &= m - 1ull;
+                    const Eval v = evaluate(sm.e[k], fpx, fpy);
+                    blend(v, sm.e[k].rgb, base + (uint32_t)k + 1u, true);
+                } else {
+                    const int k0 = (c << 6) + __builtin_ctzll(m);
+                    m &= m - 1ull;
+                    const bool two = m != 0ull;
+                    const int k1 = two ? (c << 6) + __builtin_ctzll(m) : k0;
+                    m &= m - 1ull;  // 0 stays 0
+                    const float4 cl0 = sm.e[k0].rgb, cl1 = sm.e[k1].rgb;
+                    Eval v0, v1;
+                    evaluate2(sm.e[k0], sm.e[k1], fpx, fpy, v0, v1);
+                    blend(v0, cl0, base + (uint32_t)k0 + 1u, true);
+                    blend(v1, cl1, base + (uint32_t)k1 + 1u, two);
                 }
-                T = take ? test_T : T;
-                cnt += take ? 1 : 0;
-                last = take ? base + (uint32_t)k + 1u : last;
             }
         }
     }
@@ -361,6 +407,45 @@ __device__ __forceinline__ void bwd_tile(const RasterArgs& a, int tile, BwdSmem<
     __syncthreads();
     const uint32_t stop = sm.maxlast;
 
+    // One visited entry, predicated as in the forward: its contribution is
+    // selected in or out through the factors (visited entries are finite, so a
+    // zero factor zeroes every term).
+    struct Terms {
+        float dop, aT;  // dL/d(opacity * G) times G; alpha T
+        bool contrib;
+    };
+    auto gradient = [&](const Eval& v, const float4& cl, uint32_t j) -> Terms {
+        Terms r;
+        r.contrib = j < last && v.power <= 0.0f && v.alpha >= 1.0f / 255.0f;
+        // T_i = T / (1 - alpha) as the reference recovers it
+        // (rasterizer_backward_cpu.cpp:85), with the hardware reciprocal
+        // (1 ulp): gradients need 1e-3, not bits.  alpha <= 0.99, so the
+        // reference's guard 1 - alpha > 1e-6 always holds.
+        const float Ti = T * __builtin_amdgcn_rcpf(1.0f - v.alpha);
+        float dal;
+        {
+            // gradient-only arithmetic: contracted to FMAs (the
+            // contributor decisions above stay uncontracted)
+#pragma clang fp contract(fast)
+            dal = Ti * ((cl.x - acc0) * dC0 + (cl.y - acc1) * dC1 + (cl.z - acc2) * dC2);
+        }
+        // dL/d(opacity * G) = dal * G; dL/dpower = opacity times that,
+        // and the opacity is applied once per Gaussian when the sums
+        // leave LDS (alpha >= 0.99 is the clamp: no gradient)
+        r.dop = (r.contrib && v.alpha < 0.99f) ? dal * v.ep : 0.0f;
+        r.aT = r.contrib ? v.alpha * Ti : 0.0f;
+        // colour behind the next entry: alpha c + (1 - alpha) acc
+        const float ac = r.contrib ? v.alpha : 0.0f;
+        {
+#pragma clang fp contract(fast)
+            acc0 += ac * (cl.x - acc0);
+            acc1 += ac * (cl.y - acc1);
+            acc2 += ac * (cl.z - acc2);
+        }
+        T = r.contrib ? Ti : T;
+        return r;
+    };
+
     for (uint32_t hi = stop; hi > start;) {
         const uint32_t lo = (hi - start > (uint32_t)BATCH) ? hi - BATCH : start;
         const int n = (int)(hi - lo);
@@ -390,48 +475,13 @@ __device__ __forceinline__ void bwd_tile(const RasterArgs& a, int tile, BwdSmem<
             while (bits != 0ull) {
                 const int k = (ch << 6) + (63 - __builtin_clzll(bits));
                 bits &= ~(1ull << (k & 63));
-                const uint32_t j = lo + (uint32_t)k;
-                // predicated, as the forward: every lane evaluates the entry and
-                // its contribution is selected in or out, through the factors
-                // below (visited entries are finite, so a zero factor zeroes
-                // every term)
-                const float2 m = sm.e[k].xy;
-                const float4 co = sm.e[k].co;
                 const float4 cl = sm.e[k].rgb;
-                const float dx = m.x - fpx, dy = m.y - fpy;
-                const float power = power_of(co, dx, dy);
-                float ep;
-                const float alpha = gsd::raster_alpha_wave(co.w, power, &ep);
-                const bool contrib = j < last && power <= 0.0f && alpha >= 1.0f / 255.0f;
-                const float oma = 1.0f - alpha;
-                // T_i = T / (1 - alpha) as the reference recovers it
-                // (rasterizer_backward_cpu.cpp:85), with the hardware
-                // reciprocal (1 ulp): gradients need 1e-3, not bits
-                const float Ti = (oma > 1e-6f) ? T * __builtin_amdgcn_rcpf(oma) : 0.0f;
-                float dal;
-                {
-                    // gradient-only arithmetic: contracted to FMAs (the
-                    // contributor decisions above stay uncontracted)
-#pragma clang fp contract(fast)
-                    dal = Ti * ((cl.x - acc0) * dC0 + (cl.y - acc1) * dC1 + (cl.z - acc2) * dC2);
-                }
-                // dL/d(opacity * G) = dal * G; dL/dpower = opacity times that,
-                // and the opacity is applied once per Gaussian when the sums
-                // leave LDS (alpha >= 0.99 is the clamp: no gradient)
-                const float dop = (contrib && alpha < 0.99f) ? dal * ep : 0.0f;
-                const float aT = contrib ? alpha * Ti : 0.0f;
-                // colour behind the next entry: alpha c + (1 - alpha) acc
-                const float ac = contrib ? alpha : 0.0f;
-                {
-#pragma clang fp contract(fast)
-                    acc0 += ac * (cl.x - acc0);
-                    acc1 += ac * (cl.y - acc1);
-                    acc2 += ac * (cl.z - acc2);
-                }
-                T = contrib ? Ti : T;
-                if (__ballot(contrib) != 0ull) {
-                    const float v = wave_reduce9(dop, dx, dy, aT * dC0, aT * dC1, aT * dC2, role);
-                    if (role.term >= 0 && v != 0.0f) atomicAdd(&sm.g[k][role.term], v);
+                const Eval v = evaluate(sm.e[k], fpx, fpy);
+                const Terms r = gradient(v, cl, lo + (uint32_t)k);
+                if (__ballot(r.contrib) != 0ull) {
+                    const float sum = wave_reduce9(r.dop, v.dx, v.dy, r.aT * dC0, r.aT * dC1, r.aT * dC2, role);
+                    if (role.term >= 0 && sum != 0.0f)
+                        atomicAdd(&sm.g[0][0] + (__builtin_amdgcn_readfirstlane(k * NG) + role.term), sum);
                 }
             }
         }
@@ -471,10 +521,10 @@ __device__ __forceinline__ void bwd_tile(const RasterArgs& a, int tile, BwdSmem<
     }
 }
 
-template <int BATCH>
+template <int BATCH, bool PAIR>
 __global__ __launch_bounds__(256) void raster_fwd_kernel(RasterArgs a, PixOut o) {
     __shared__ FwdSmem<BATCH> sm;
-    fwd_tile<BATCH>(a, gsd::xcd_remap(blockIdx.x, gridDim.x), sm, o);
+    fwd_tile<BATCH, PAIR>(a, gsd::xcd_remap(blockIdx.x, gridDim.x), sm, o);
 }
 
 template <int BATCH>
@@ -561,7 +611,7 @@ __global__ __launch_bounds__(256) void raster_fwd_multi_kernel(MultiRaster m, Mu
         RasterArgs a = view_args(m, v);
         const size_t p0 = (size_t)m.pix_off[v];
         PixOut po{o.img + p0 * 3, o.T_final + p0, o.n_contrib + p0, o.last_contrib + p0};
-        fwd_tile<BATCH>(a, g - m.views[v].w, sm, po);
+        fwd_tile<BATCH, false>(a, g - m.views[v].w, sm, po);
     }
 }
 
@@ -589,11 +639,21 @@ hipError_t launch_raster_fwd(const RasterArgs& a, int num_tiles, int batch, floa
                              uint32_t* last_contrib, hipStream_t s) {
     if (num_tiles <= 0) return hipSuccess;
     PixOut o{img, T_final, n_contrib, last_contrib};
+    // Up to 1024 tiles (four waves per SIMD) a wave's own instruction chain sets
+    // the pace, and two entries at a time overlap it: 43 -> 36 us at 256 tiles
+    // (10k Gaussians), 70 -> 62 us at 520; from 3400 tiles on it is a draw.
+    const bool pair = num_tiles <= 1024;
     switch (batch) {
-        case 64: raster_fwd_kernel<64><<<num_tiles, 256, 0, s>>>(a, o); break;
-        case 128: raster_fwd_kernel<128><<<num_tiles, 256, 0, s>>>(a, o); break;
-        case 256: raster_fwd_kernel<256><<<num_tiles, 256, 0, s>>>(a, o); break;
-        case 512: raster_fwd_kernel<512><<<num_tiles, 256, 0, s>>>(a, o); break;
+#define FWD(B)                                                              \
+    case B:                                                                 \
+        if (pair) raster_fwd_kernel<B, true><<<num_tiles, 256, 0, s>>>(a, o); \
+        else raster_fwd_kernel<B, false><<<num_tiles, 256, 0, s>>>(a, o);   \
+        break
+        FWD(64);
+        FWD(128);
+        FWD(256);
+        FWD(512);
+#undef FWD
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
