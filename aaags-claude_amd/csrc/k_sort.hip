@@ -33,6 +33,11 @@ constexpr int RS_WAVES = RS_THREADS / 64;
 // runs per digit), 1024 below 4M keys so that a sort of ~1M keys still spreads
 // over ~1000 blocks instead of ~250.
 constexpr uint32_t RS_SMALL_LIMIT = 1u << 22;
+// Sorts of at most this many blocks scan the digit counts inside the scatter
+// (rs_downsweep_kernel, DIRECT): 58.7 -> 53.2 us at 50k keys and four passes,
+// 59.5 -> 50.4 at 100k; at 98 blocks (200k keys) it is a draw (62.1, 62.4), at
+// 147 a loss (64.7 -> 75.8).
+constexpr uint32_t RS_DIRECT_BLOCKS = 64;
 
 // n_dev (optional): the item count lives on the device (graph capture); the
 // launch is sized for n (the capacity) and the kernels use min(*n_dev, n).
@@ -363,7 +368,9 @@ __global__ __launch_bounds__(256) void tile_ranges_multi_kernel(const uint64_t* 
 }
 
 // ---------------------------------------------------------- radix sort ----
-template <int BITS, int ROUNDS>
+// BLOCK_MAJOR: counts at hist[block][digit] (sorts of at most RS_DIRECT_BLOCKS
+// blocks), else digit-major rows hs apart.
+template <int BITS, int ROUNDS, bool BLOCK_MAJOR>
 __global__ __launch_bounds__(RS_THREADS) void rs_upsweep_kernel(const uint64_t* __restrict__ keys, uint32_t n_cap,
                                                                 const uint32_t* __restrict__ n_dev, int shift,
                                                                 uint32_t hs, uint32_t* __restrict__ hist) {
@@ -398,7 +405,7 @@ __global__ __launch_bounds__(RS_THREADS) void rs_upsweep_kernel(const uint64_t* 
         uint32_t s = 0;
 #pragma unroll
         for (int k = 0; k < RS_WAVES; k++) s += s_h[k][d];
-        hist[(size_t)d * hs + blockIdx.x] = s;
+        hist[BLOCK_MAJOR ? (size_t)blockIdx.x * RADIX + d : (size_t)d * hs + blockIdx.x] = s;
     }
 }
 
@@ -446,7 +453,11 @@ __global__ __launch_bounds__(64) void rs_digit_scan_kernel(const uint32_t* __res
 }
 
 // VALS = false sorts self-contained 64-bit words (no separate value array).
-template <int BITS, bool VALS, int ROUNDS>
+// DIRECT: goff holds the block-major counts of `hs` blocks themselves, and each
+// block adds up the digits of the blocks before it and of all blocks on its
+// own: at most RS_DIRECT_BLOCKS independent loads per thread, instead of a
+// launch in between (4 us each, four per depth sort).
+template <int BITS, bool VALS, int ROUNDS, bool DIRECT>
 __global__ __launch_bounds__(RS_THREADS) void rs_downsweep_kernel(const uint64_t* __restrict__ keys_in,
                                                                   const uint32_t* __restrict__ vals_in, uint32_t n_cap,
                                                                   const uint32_t* __restrict__ n_dev, int shift,
@@ -471,10 +482,23 @@ __global__ __launch_bounds__(RS_THREADS) void rs_downsweep_kernel(const uint64_t
         // the digit's start in the output: all smaller digits, then this
         // digit's keys in the blocks before this one
         static_assert(RADIX <= RS_THREADS, "one digit per thread");
-        const uint32_t t = threadIdx.x < RADIX ? dtot[threadIdx.x] : 0u;
+        uint32_t t = 0u, before = 0u;
+        if (DIRECT) {
+            if (threadIdx.x < RADIX) {
+#pragma unroll 16
+                for (uint32_t b = 0; b < hs; b++) {
+                    const uint32_t c = goff[(size_t)b * RADIX + threadIdx.x];
+                    t += c;
+                    before += b < blockIdx.x ? c : 0u;
+                }
+            }
+        } else if (threadIdx.x < RADIX) {
+            t = dtot[threadIdx.x];
+            before = goff[(size_t)threadIdx.x * hs + blockIdx.x];
+        }
         uint32_t total;
         const uint32_t ex = block_exclusive_scan<uint32_t>(t, s_scan, &total);
-        if (threadIdx.x < RADIX) s_goff[threadIdx.x] = ex + goff[(size_t)threadIdx.x * hs + blockIdx.x];
+        if (threadIdx.x < RADIX) s_goff[threadIdx.x] = ex + before;
     }
     __syncthreads();
 
@@ -554,6 +578,96 @@ __global__ __launch_bounds__(RS_THREADS) void rs_downsweep_kernel(const uint64_t
             keys_out[g] = k;
             if constexpr (VALS) vals_out[g] = s_v[p];
         }
+    }
+}
+
+// ------------------------------------------------------ one workgroup ----
+// Sorts of at most RS_SINGLE_MAX self-contained words: one workgroup holds all
+// of them, in registers between the passes and in LDS for the exchange, so a
+// sort is one launch instead of two or three per pass (launches set the pace at
+// this size: 57 us in twelve launches for 10k words, now 34).
+constexpr int RS1_THREADS = 1024, RS1_WAVES = RS1_THREADS / 64;
+constexpr uint32_t RS_SINGLE_MAX = 16u * RS1_THREADS;
+
+struct SinglePasses {
+    int n;
+    int shift[8];
+};
+
+template <int BITS, int ITEMS>
+__global__ __launch_bounds__(RS1_THREADS) void rs_single_kernel(const uint64_t* __restrict__ keys_in, uint32_t n_cap,
+                                                                const uint32_t* __restrict__ n_dev, SinglePasses ps,
+                                                                uint64_t* __restrict__ keys_out) {
+    constexpr int RADIX = 1 << BITS;
+    const uint32_t n = live_count(n_cap, n_dev);
+    __shared__ uint64_t s_k[RS1_THREADS * ITEMS];
+    __shared__ uint32_t s_wh[RS1_WAVES][RADIX];
+    __shared__ uint32_t s_dstart[RADIX];
+    __shared__ uint32_t s_scan[RS1_WAVES];
+    const int w = threadIdx.x >> 6, l = lane_id();
+    const uint32_t wbase = (uint32_t)w * (ITEMS * 64);
+    uint64_t k_r[ITEMS];
+    uint32_t rank_r[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; r++) {
+        const uint32_t i = wbase + r * 64 + l;
+        k_r[r] = i < n ? keys_in[i] : 0ull;
+    }
+    for (int pass = 0; pass < ps.n; pass++) {
+        const int shift = ps.shift[pass];
+        for (int i = threadIdx.x; i < RS1_WAVES * RADIX; i += RS1_THREADS) (&s_wh[0][0])[i] = 0u;
+        __syncthreads();
+        // per-wave stable ranks: rounds in key order, lanes in key order
+#pragma unroll
+        for (int r = 0; r < ITEMS; r++) {
+            const bool valid = wbase + r * 64 + l < n;
+            const uint64_t active = __ballot(valid);
+            rank_r[r] = 0u;
+            if (active != 0) {
+                const uint32_t d = digit_of<BITS>(k_r[r], shift);
+                const uint64_t peers = match_digit<BITS>(d, active);
+                uint32_t before = 0u;
+                if (valid) before = s_wh[w][d];
+                __builtin_amdgcn_wave_barrier();
+                if (valid && (peers & lanemask_lt()) == 0) s_wh[w][d] = before + (uint32_t)__popcll(peers);
+                __builtin_amdgcn_wave_barrier();
+                rank_r[r] = before + (uint32_t)__popcll(peers & lanemask_lt());
+            }
+        }
+        __syncthreads();
+        // digit totals, per-wave offsets inside each digit, digit starts
+        uint32_t tot = 0u;
+        if (threadIdx.x < RADIX) {
+#pragma unroll
+            for (int k = 0; k < RS1_WAVES; k++) {
+                const uint32_t c = s_wh[k][threadIdx.x];
+                s_wh[k][threadIdx.x] = tot;
+                tot += c;
+            }
+        }
+        uint32_t total;
+        const uint32_t ex = block_exclusive_scan<uint32_t>(tot, s_scan, &total);
+        if (threadIdx.x < RADIX) s_dstart[threadIdx.x] = ex;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < ITEMS; r++) {
+            if (wbase + r * 64 + l < n) {
+                const uint32_t d = digit_of<BITS>(k_r[r], shift);
+                s_k[s_dstart[d] + s_wh[w][d] + rank_r[r]] = k_r[r];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < ITEMS; r++) {
+            const uint32_t i = wbase + r * 64 + l;
+            if (i < n) k_r[r] = s_k[i];
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int r = 0; r < ITEMS; r++) {
+        const uint32_t i = wbase + r * 64 + l;
+        if (i < n) keys_out[i] = k_r[r];
     }
 }
 
@@ -1000,20 +1114,31 @@ static hipError_t onesweep_sort(const uint64_t* ki, const uint32_t* vi, uint64_t
     return hipGetLastError();
 }
 
+template <int BITS, int ROUNDS, bool DIRECT>
+static hipError_t sort_pass_d(const uint64_t* ki, const uint32_t* vi, uint64_t* ko, uint32_t* vo, uint32_t n,
+                              const uint32_t* n_dev, int shift, uint32_t* hist, uint32_t* goff,
+                              uint32_t* dtot, hipStream_t s) {
+    const uint32_t nb = radix_blocks(n), hs = radix_row_stride(nb);
+    rs_upsweep_kernel<BITS, ROUNDS, DIRECT><<<nb, RS_THREADS, 0, s>>>(ki, n, n_dev, shift, hs, hist);
+    if (!DIRECT) rs_digit_scan_kernel<<<1u << BITS, 64, 0, s>>>(hist, nb, hs, goff, dtot);
+    const uint32_t stride = DIRECT ? nb : hs;
+    const uint32_t* counts = DIRECT ? hist : goff;
+    if (vi)
+        rs_downsweep_kernel<BITS, true, ROUNDS, DIRECT>
+            <<<nb, RS_THREADS, 0, s>>>(ki, vi, n, n_dev, shift, stride, counts, dtot, ko, vo);
+    else
+        rs_downsweep_kernel<BITS, false, ROUNDS, DIRECT>
+            <<<nb, RS_THREADS, 0, s>>>(ki, nullptr, n, n_dev, shift, stride, counts, dtot, ko, nullptr);
+    return hipGetLastError();
+}
+
 template <int BITS, int ROUNDS>
 static hipError_t sort_pass_r(const uint64_t* ki, const uint32_t* vi, uint64_t* ko, uint32_t* vo, uint32_t n,
                               const uint32_t* n_dev, int shift, uint32_t* hist, uint32_t* goff,
                               uint32_t* dtot, hipStream_t s) {
-    const uint32_t nb = radix_blocks(n), hs = radix_row_stride(nb);
-    rs_upsweep_kernel<BITS, ROUNDS><<<nb, RS_THREADS, 0, s>>>(ki, n, n_dev, shift, hs, hist);
-    rs_digit_scan_kernel<<<1u << BITS, 64, 0, s>>>(hist, nb, hs, goff, dtot);
-    if (vi)
-        rs_downsweep_kernel<BITS, true, ROUNDS>
-            <<<nb, RS_THREADS, 0, s>>>(ki, vi, n, n_dev, shift, hs, goff, dtot, ko, vo);
-    else
-        rs_downsweep_kernel<BITS, false, ROUNDS>
-            <<<nb, RS_THREADS, 0, s>>>(ki, nullptr, n, n_dev, shift, hs, goff, dtot, ko, nullptr);
-    return hipGetLastError();
+    if (radix_blocks(n) <= RS_DIRECT_BLOCKS)
+        return sort_pass_d<BITS, ROUNDS, true>(ki, vi, ko, vo, n, n_dev, shift, hist, goff, dtot, s);
+    return sort_pass_d<BITS, ROUNDS, false>(ki, vi, ko, vo, n, n_dev, shift, hist, goff, dtot, s);
 }
 
 template <int BITS>
@@ -1023,6 +1148,27 @@ static hipError_t sort_pass(const uint64_t* ki, const uint32_t* vi, uint64_t* ko
     if (radix_rounds(n) == 16) return sort_pass_r<BITS, 16>(ki, vi, ko, vo, n, n_dev, shift, hist, goff, dtot, s);
     if (radix_rounds(n) == 8) return sort_pass_r<BITS, 8>(ki, vi, ko, vo, n, n_dev, shift, hist, goff, dtot, s);
     return sort_pass_r<BITS, 4>(ki, vi, ko, vo, n, n_dev, shift, hist, goff, dtot, s);
+}
+
+static hipError_t single_sort(const uint64_t* ki, uint64_t* ko, uint32_t n, const uint32_t* n_dev, const int* shifts,
+                              int passes, hipStream_t s) {
+    SinglePasses ps{};
+    ps.n = passes;
+    for (int p = 0; p < passes; p++) ps.shift[p] = shifts[p];
+    switch ((n + 2u * RS1_THREADS - 1) / (2u * RS1_THREADS)) {  // as few rounds as hold the words
+#define RS1(I) case I: rs_single_kernel<8, 2 * I><<<1, RS1_THREADS, 0, s>>>(ki, n, n_dev, ps, ko); break
+        RS1(1);
+        RS1(2);
+        RS1(3);
+        RS1(4);
+        RS1(5);
+        RS1(6);
+        RS1(7);
+        RS1(8);
+#undef RS1
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
 }
 
 // Stable LSD sort of n keys (with optional uint32 values) on key bits
@@ -1063,6 +1209,8 @@ hipError_t launch_radix_sort_bits(const uint64_t* keys_in, const uint32_t* vals_
         if (shift + radix_bits > end_bit && end_bit - radix_bits >= begin_bit) shift = end_bit - radix_bits;
         shifts[p] = shift;
     }
+    if (!vals && radix_bits == 8 && n <= RS_SINGLE_MAX && passes <= 8)
+        return single_sort(keys_in, keys_out, n, n_dev, shifts, passes, s);
     if (use_onesweep(n, passes)) {
         switch (radix_bits) {
             case 4: return onesweep_sort<4>(keys_in, vals_in, keys_out, vals_out, pk, pv, n, n_dev, shifts, passes,
