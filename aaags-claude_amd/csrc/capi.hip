@@ -499,7 +499,26 @@ extern "C" int gs_ctx_apply_tuning(gs_ctx* c, const gs_tuning* t) {
     return GS_OK;
 }
 
-// Room for at least `records` bin records.
+// First guess for the record buffer, in records per Gaussian (6 at 1M
+// Gaussians and 1080p).  That many lie behind the binning's tables in its
+// workspace, so most contexts allocate nothing more; a view that needs more
+// gets a buffer of its own, which then stays.
+constexpr size_t kRecordsPerGaussian = 8;
+
+size_t gs_bin_guess_bytes(const gsb::BinArgs& a) {
+    return (size_t)a.V * a.N * kRecordsPerGaussian * bin_record_bytes(a) + 256;
+}
+
+// Record buffer for the binning whose workspace ends with `guess`
+// (gs_bin_guess_bytes): that, or the context's own buffer where that is larger.
+static void coarse_set(gs_ctx* c, gsb::BinArgs& a, void* guess) {
+    const size_t each = bin_record_bytes(a), have = gs_bin_guess_bytes(a) - 256;
+    const bool own = c->coarse_bytes > have;
+    a.coarse = own ? c->coarse : guess;
+    a.coarse_cap = (uint32_t)std::min<size_t>((own ? c->coarse_bytes : have) / each, 0xFFFFFFFFu);
+}
+
+// A buffer of the context's own for at least `records` bin records.
 static int coarse_get(gs_ctx* c, size_t records, gsb::BinArgs& a) {
     const size_t each = bin_record_bytes(a);
     int st = grow(c, &c->coarse, &c->coarse_bytes, records * each, &a.coarse);
@@ -517,18 +536,14 @@ int gs_bin_fits(gs_ctx* c, const gsb::BinArgs& a, unsigned long long records, bo
     return coarse_get(c, (size_t)records, grown);
 }
 
-// First guess for the record buffer, in records per Gaussian (6 at 1M
-// Gaussians and 1080p; a view that needs more grows it once).
-constexpr size_t kRecordsPerGaussian = 8;
-
-int gs_bin_count(gs_ctx* c, gsb::BinArgs& a, unsigned long long* pairs) {
+int gs_bin_count(gs_ctx* c, gsb::BinArgs& a, void* guess, unsigned long long* pairs) {
     void* sm;
     int st = gs_small_get(c, &sm);
     if (st) return st;
     // {pairs, records} side by side: one copy reads both
     unsigned long long* counts = reinterpret_cast<unsigned long long*>(static_cast<char*>(sm) + GS_SMALL_TOTAL64);
     a.overflow = reinterpret_cast<uint32_t*>(static_cast<char*>(sm) + GS_SMALL_OVERFLOW);
-    if ((st = coarse_get(c, (size_t)a.V * a.N * kRecordsPerGaussian, a))) return st;
+    coarse_set(c, a, guess);
     unsigned long long got[2] = {0, 0};
     for (int attempt = 0;; attempt++) {
         GS_HIP(launch_bin_lists(a, c->stream, counts + 1, nullptr, counts, attempt > 0), "binning kernels");
@@ -578,7 +593,7 @@ int gs_bin_prepare(gs_ctx* c, int n, const gs_preprocessed* pre, int width, int 
     const size_t un = (size_t)n;
     void* ws2;
     if ((st = gs_ws2_get(c, 2 * al(un * 8) + al(un * 4) + radix_workspace_bytes((uint32_t)n, c->radix_bits) +
-                                bin_workspace_bytes(a),
+                                bin_workspace_bytes(a) + gs_bin_guess_bytes(a),
                          &ws2)))
         return st;
     char* w = static_cast<char*>(ws2);
@@ -587,6 +602,7 @@ int gs_bin_prepare(gs_ctx* c, int n, const gs_preprocessed* pre, int width, int 
     uint32_t* rect_idx = reinterpret_cast<uint32_t*>(w); w += al(un * 4);  // packed rectangles, index order
     void* dsort_ws = w;
     bin_carve(a, w + radix_workspace_bytes((uint32_t)n, c->radix_bits));
+    void* guess = w + radix_workspace_bytes((uint32_t)n, c->radix_bits) + al(bin_workspace_bytes(a));
     GS_HIP(launch_depth_words(n, pre->depths, pre->radii, dkeys, c->stream, pre->means2D, gx, gy, rect_idx),
            "depth keys kernel");
     GS_HIP(launch_radix_sort_bits(dkeys, nullptr, dkeys_s, nullptr, (uint32_t)n, 0, 32, c->radix_bits, dsort_ws,
@@ -599,12 +615,12 @@ int gs_bin_prepare(gs_ctx* c, int n, const gs_preprocessed* pre, int width, int 
         void* sm;
         if ((st = gs_small_get(c, &sm))) return st;
         a.overflow = reinterpret_cast<uint32_t*>(static_cast<char*>(sm) + GS_SMALL_OVERFLOW);
-        if ((st = coarse_get(c, un * kRecordsPerGaussian, a))) return st;
+        coarse_set(c, a, guess);
         GS_HIP(launch_bin_lists(a, c->stream, host_counts + 1, nullptr, host_counts), "binning kernels");
         if (ev_total) GS_HIP(hipEventRecord(ev_total, c->stream), "hipEventRecord");
     } else {
         unsigned long long K = 0;
-        if ((st = gs_bin_count(c, a, &K))) return st;
+        if ((st = gs_bin_count(c, a, guess, &K))) return st;
         if (pairs) *pairs = (long long)K;
     }
     c->bin_pending = true;

@@ -37,7 +37,7 @@ struct gs_ctx {
     int bin_tpl = 1;
     int persistent_per_cu = 6;  // batched raster: persistent groups per CU (0: one group per tile)
     int split_groups = 64;      // likewise: the forward no longer runs in two rounds
-    void* coarse = nullptr;     // the binning's bin records
+    void* coarse = nullptr;     // bin records of a binning whose first guess was too small
     size_t coarse_bytes = 0;
     gsb::BinArgs* bin = nullptr;  // the binning that gs_bin_prepare left for gs_bin_finish
     bool bin_pending = false;
@@ -70,7 +70,9 @@ int gs_bin_prepare(gs_ctx* c, int n, const gs_preprocessed* pre, int width, int 
 int gs_bin_finish(gs_ctx* c, uint32_t* values, uint32_t capacity, uint32_t* ranges);
 // The same two halves over prepared arguments (order, sizes, views, rectangles
 // or means set; the workspace carved), for the eval_3D binning.
-int gs_bin_count(gs_ctx* c, gsb::BinArgs& a, unsigned long long* pairs);
+// guess: gs_bin_guess_bytes of workspace for the records.
+int gs_bin_count(gs_ctx* c, gsb::BinArgs& a, void* guess, unsigned long long* pairs);
+size_t gs_bin_guess_bytes(const gsb::BinArgs& a);
 // Whether `records` bin records fit the context's buffer; grows it if not.
 int gs_bin_fits(gs_ctx* c, const gsb::BinArgs& a, unsigned long long records, bool* fits);
 extern "C" int gs_check_overflow(gs_ctx* c, int* overflowed);

@@ -1063,7 +1063,7 @@ extern "C" int gs_bin_tiles_3d(gs_ctx* c, int n, const gs_preprocessed* pre, con
     const size_t np = scan_partials_needed((uint32_t)num_tiles + 1) + 1;
     void* ws2;
     if ((st = gs_ws2_get(c, alg(bin_workspace_bytes(a)) + alg(np * 8) + alg((size_t)num_tiles * 16) +
-                                2 * alg(((size_t)num_tiles + 1) * 4) + alg(un * 64),
+                                2 * alg(((size_t)num_tiles + 1) * 4) + alg(un * 64) + gs_bin_guess_bytes(a),
                          &ws2)))
         return st;
     char* w = static_cast<char*>(ws2);
@@ -1072,13 +1072,13 @@ extern "C" int gs_bin_tiles_3d(gs_ctx* c, int n, const gs_preprocessed* pre, con
     float4* rays = reinterpret_cast<float4*>(w); w += alg((size_t)num_tiles * 16);
     uint32_t* bigcnt = reinterpret_cast<uint32_t*>(w); w += alg(((size_t)num_tiles + 1) * 4);
     uint32_t* boff = reinterpret_cast<uint32_t*>(w); w += alg(((size_t)num_tiles + 1) * 4);
-    float4* packed = reinterpret_cast<float4*>(w);
+    float4* packed = reinterpret_cast<float4*>(w); w += alg(un * 64);
     if (k.have_ivp) {
         gs3::tile_rays_kernel<<<(num_tiles + 255) / 256, 256, 0, c->stream>>>(k, rays);
         G3_HIP(hipGetLastError(), "tile rays kernel");
     }
     unsigned long long K = 0;
-    if ((st = gs_bin_count(c, a, &K))) return st;
+    if ((st = gs_bin_count(c, a, w, &K))) return st;
     if (total) *total = (long long)K;
     if (K > capacity)
         return gs_set_error(GS_ERR_CAPACITY, "gs_bin_tiles_3d: %llu pairs exceed capacity %u", K, capacity);
