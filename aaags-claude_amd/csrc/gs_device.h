@@ -43,9 +43,8 @@ static const uint64_t kExp2TabHost[32] = GS_EXP2_TAB;
 // exp_ref with the 2^(i/32) table at `tab` (a copy of GS_EXP2_TAB, e.g. in LDS:
 // the table index differs from lane to lane, so a copy in LDS saves a global
 // load's latency per call in loops that evaluate many exponentials).
-__host__ __device__ __forceinline__ float exp_ref_tab(float x, const uint64_t* tab) {
-    if (!(x <= 0x1.62e42ep6f)) return x != x ? x + x : __builtin_inff();  // NaN, overflow
-    if (x < -0x1.9fe368p6f) return 0.0f;                                   // below 2^-150
+// exp_ref_core: its arithmetic, without the range checks.
+__host__ __device__ __forceinline__ float exp_ref_core(float x, const uint64_t* tab) {
     constexpr double kInvLn2N = 0x1.71547652b82fep+0 * 32.0, kShift = 0x1.8p+52;
     constexpr double kC0 = 0x1.c6af84b912394p-5 / 32 / 32 / 32, kC1 = 0x1.ebfce50fac4f3p-3 / 32 / 32,
                      kC2 = 0x1.62e42ff0c52d6p-1 / 32;
@@ -63,6 +62,18 @@ __host__ __device__ __forceinline__ float exp_ref_tab(float x, const uint64_t* t
     double y = __builtin_fma(kC2, r, 1.0);
     y = __builtin_fma(z, r2, y);
     return (float)(y * sc);
+}
+
+__host__ __device__ __forceinline__ float exp_ref_tab(float x, const uint64_t* tab) {
+    if (!(x <= 0x1.62e42ep6f)) return x != x ? x + x : __builtin_inff();  // NaN, overflow
+    if (x < -0x1.9fe368p6f) return 0.0f;                                   // below 2^-150
+    return exp_ref_core(x, tab);
+}
+
+// The same for an x that is not positive, or NaN: one select, no branch.
+__host__ __device__ __forceinline__ float exp_ref_nonpos(float x, const uint64_t* tab) {
+    const float v = exp_ref_core(x, tab);
+    return x < -0x1.9fe368p6f ? 0.0f : v;
 }
 
 __host__ __device__ __forceinline__ float exp_ref(float x) {

@@ -14,11 +14,11 @@
 // Layout in HBM (the reference's PreprocessOutput arrays): gauss2screen
 // [N][16] row-major, cov3D_inv [N][6] (upper triangle), mean_offset [N][3].
 // The rasterizer stages rows 0, 1 and 3 of gauss2screen, the inverse
-// covariance, the mean offset, opacity and view depth of 256 Gaussians at a
-// time in LDS (112 B each); every lane of the tile's workgroup evaluates its
-// pixel against each staged entry and keeps its 16 nearest entries (by depth
-// along its own ray) sorted in a ring in LDS, blending the front one whenever
-// a 17th arrives.
+// covariance, the mean offset, opacity and view depth of 64 Gaussians at a time
+// in LDS (96 B each); every lane of the tile's workgroup marks the entries that
+// reach its pixel and evaluates those, and keeps its 16 nearest entries (by
+// depth along its own ray) in order, their depths in registers, blending the
+// front one whenever a 17th arrives.
 #include <cmath>
 #include <cstring>
 
@@ -525,24 +525,108 @@ struct Entry3 {
     float mo[3];
     float op, depth;
     uint32_t id;
-    float cut;  // 1e-3 - ln(1 / (255 op)): half the squared distance beyond which alpha < 1/255
-    float pad[3];
 };
-static_assert(sizeof(Entry3) == 112, "one LDS record per Gaussian");
+static_assert(sizeof(Entry3) == 96, "one LDS record per Gaussian");
 
-// Entries staged per round.  The k-buffers take 48 KB of LDS per workgroup;
-// 32 staged entries (3.5 KB) keep a workgroup at 52 KB, so three fit a CU
-// (256 entries, 28 KB, allowed two): the kernel is latency-bound, and the third
-// workgroup per CU hides more than the extra staging rounds cost
-// (3.75 -> 2.82 ms at 1M Gaussians, 1080p).
-constexpr int R3_BATCH = 32;
+// Entries staged per round: one wave loads them, one bit each in a lane's hit
+// mask.  The k-buffers' alphas and ids take 32 KB of LDS per workgroup, the
+// staged entries 6 KB and their reach 1.5 KB: 40 KB, so that four workgroups
+// fit a CU.
+constexpr int R3_BATCH = 64;
+constexpr int R3_GROUP = 8;  // k-buffer places that an insertion passes at a time (2: 1.99 ms, 4: 1.75, 8: 1.73)
+static_assert(KBUF % R3_GROUP == 0, "whole groups");
 
-// One workgroup per 16x16 tile, one pixel per lane (rasterizer_cpu.cpp:61-135).
-// Each lane's k-buffer is a 16-slot ring in LDS (slot-major, so the lanes of
-// a wave touch consecutive words): the front entry leaves by advancing the
-// head, and an entry is inserted from the back, moving only the deeper
-// entries.  The pairs arrive in order of depth at the tile's centre, so the
-// move count is usually zero or one.
+// The pixels of a tile that a staged entry can reach, as one quadratic in the
+// pixel's offset (x, y) from the tile's centre, |x|, |y| <= 7.5:
+//   reach(x, y) = k00 + x (k01 + x k11 + y k12) + y (k02 + y k22)
+// is positive only where the evaluation skips the entry, and its sign is all
+// that is read.  The ray of a pixel is where two planes p = r0 - fx r3 and
+// q = r1 - fy r3 meet; its squared distance is |m|^2 / |d|^2 with d = p x q and
+// m = p_w q - q_w p, both linear in (x, y) (their xy terms cancel), so
+// |m|^2 > K |d|^2 is such a quadratic: six instructions a pixel where the planes
+// and cross products take fifty.  K is twice 1e-3 + ln(255 op): alpha stays
+// below e^-0.001 / 255, which the evaluation's own rounding (1e-6) cannot lift
+// to 1/255.  The constant is lowered by what rounding can do, so that a positive
+// value is a proof (u = 2^-24):
+//  - the evaluation's m and d differ from the linear forms' by at most 16 u Em
+//    and 16 u Ed, the sums of the absolute products that enter them;
+//  - with s = 16 u (Em + sqrt(K) Ed), |m| >= sqrt(K) |d| + s follows from
+//    |m|^2 >= K (1 + 1/256) |d|^2 + 257 s^2;
+//  - the coefficients' and the quadratic's own rounding is below
+//    32 u (Nm^2 + K Nd^2), Nm and Nd bounding |m| and |d| over the tile;
+//  - 1e-30 keeps |m|^2 away from where products underflow; coefficients that
+//    could overflow, and infinities and NaN anywhere, leave the entry in reach.
+struct Reach {
+    float k00, k01, k02, k11, k12, k22;
+};
+
+__device__ __forceinline__ Reach reach_of(const float4& r0, const float4& r1, const float4& r3, float op, float X0,
+                                          float Y0) {
+#pragma clang fp contract(fast)
+    // half the squared distance beyond which alpha < 1/255, and 1e-3 more
+    const float cut = 1e-3f + __logf(255.0f * op);
+    const float u = 5.9604645e-8f;
+    const float P[4] = {r0.x - X0 * r3.x, r0.y - X0 * r3.y, r0.z - X0 * r3.z, r0.w - X0 * r3.w};
+    const float Q[4] = {r1.x - Y0 * r3.x, r1.y - Y0 * r3.y, r1.z - Y0 * r3.z, r1.w - Y0 * r3.w};
+    const float R[4] = {r3.x, r3.y, r3.z, r3.w};
+    float D0[3], D1[3], D2[3], M0[3], M1[3], M2[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const int i = (k + 1) % 3, j = (k + 2) % 3;
+        D0[k] = P[i] * Q[j] - P[j] * Q[i];
+        D1[k] = R[j] * Q[i] - R[i] * Q[j];
+        D2[k] = P[j] * R[i] - P[i] * R[j];
+        M0[k] = P[3] * Q[k] - Q[3] * P[k];
+        M1[k] = Q[3] * R[k] - R[3] * Q[k];
+        M2[k] = R[3] * P[k] - P[3] * R[k];
+    }
+    const float K = cut > 0.0f ? 2.0002f * cut : (cut <= 0.0f ? 0.0f : cut);  // NaN stays NaN
+    const float K1 = K * (1.0f + 1.0f / 256.0f);
+    auto dot = [](const float* a, const float* b) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; };
+    auto mag = [](const float* a) { return fabsf(a[0]) + fabsf(a[1]) + fabsf(a[2]); };
+    const float FX = X0 + 8.0f, FY = Y0 + 8.0f;
+    const float a012 = mag(&r0.x) + FX * mag(&r3.x), b012 = mag(&r1.x) + FY * mag(&r3.x);
+    const float a3 = fabsf(r0.w) + FX * fabsf(r3.w), b3 = fabsf(r1.w) + FY * fabsf(r3.w);
+    const float Ed = a012 * b012, Em = a3 * b012 + a012 * b3;
+    const float s = 16.0f * u * (Em + sqrtf(K) * Ed);
+    const float Nm = mag(M0) + 8.0f * (mag(M1) + mag(M2)), Nd = mag(D0) + 8.0f * (mag(D1) + mag(D2));
+    const float slack = 257.0f * s * s + 32.0f * u * (Nm * Nm + K1 * (Nd * Nd)) + 1e-30f;
+    Reach k;
+    k.k00 = (dot(M0, M0) - K1 * dot(D0, D0)) - slack;
+    k.k01 = 2.0f * (dot(M0, M1) - K1 * dot(D0, D1));
+    k.k02 = 2.0f * (dot(M0, M2) - K1 * dot(D0, D2));
+    k.k12 = 2.0f * (dot(M1, M2) - K1 * dot(D1, D2));
+    k.k11 = dot(M1, M1) - K1 * dot(D1, D1);
+    k.k22 = dot(M2, M2) - K1 * dot(D2, D2);
+    const float top = fmaxf(fmaxf(fabsf(k.k01) + fabsf(k.k02), fabsf(k.k11) + fabsf(k.k12)), fabsf(k.k22));
+    if (!(Em < 1e18f && Ed < 1e18f && fabsf(k.k00) < 1e30f && top < 1e30f)) {
+        k.k00 = -1.0f;
+        k.k01 = k.k02 = k.k11 = k.k12 = k.k22 = 0.0f;
+    }
+    return k;
+}
+
+// One workgroup per 16x16 tile, one pixel per lane (rasterizer_cpu.cpp:61-135);
+// a wave takes an 8x8 block of the tile.
+// Each lane keeps the depths of its k-buffer in 16 registers, in order, and in a
+// 64-bit word which of its 16 LDS slots (slot-major, so the lanes of a wave touch
+// consecutive words) holds each one's alpha and id.  An insertion is the same few
+// instructions in every lane, where moving the deeper entries up one by one
+// through LDS waited for as many dependent reads as the wave's busiest lane
+// needed, and a third workgroup's worth of LDS is free for a fourth workgroup.
+//
+// What bounds it is the issue of vector instructions: a pixel blends 73 of the
+// 330 entries that its tile visits (1M Gaussians, 1080p), at some 230
+// instructions an evaluation.  Every staged round therefore goes in two steps.
+// All lanes first mark the entries that reach their pixel (reach_of), then each
+// lane takes its own marked entries in order, so that a wave makes as many
+// evaluations as its busiest lane needs (116 of 87 on average with 32 staged
+// entries, fewer with 64) and not one for every entry that any lane needs.  The
+// next round's entries are loaded while this one is evaluated, and a blended
+// colour is added when the next one blends, so that neither load is waited for.
+// Measured there: 3.45 ms evaluating entry by entry with the k-buffer a ring in
+// LDS, 3.17 ms with the marks, 2.01 ms with the depths in registers, 1.85 ms with
+// insertions by groups, 1.73 ms with 64 staged entries.
 __global__ __launch_bounds__(256) void raster3d_kernel(Cam3 c, const uint32_t* __restrict__ ranges,
                                                        const uint32_t* __restrict__ values,
                                                        const float* __restrict__ g2s, const float* __restrict__ cinv,
@@ -551,7 +635,8 @@ __global__ __launch_bounds__(256) void raster3d_kernel(Cam3 c, const uint32_t* _
                                                        float bg0, float bg1, float bg2, float* __restrict__ img,
                                                        float* __restrict__ T_final, int* __restrict__ n_contrib) {
     __shared__ Entry3 sm[R3_BATCH];
-    __shared__ float s_kd[KBUF][256];
+    __shared__ float4 s_q0[R3_BATCH];  // k00, k01, k02, k11
+    __shared__ float2 s_q1[R3_BATCH];  // k12, k22
     __shared__ float s_ka[KBUF][256];
     __shared__ uint32_t s_ki[KBUF][256];
     __shared__ uint64_t s_e2[32];  // exp_ref's table (read before the first barrier below)
@@ -559,126 +644,195 @@ __global__ __launch_bounds__(256) void raster3d_kernel(Cam3 c, const uint32_t* _
     const int tx = tile % c.gx, ty = tile / c.gx;
     const int t = threadIdx.x;
     if (t < 32) s_e2[t] = kExp2TabDev[t];
-    const int px = tx * 16 + (t & 15), py = ty * 16 + (t >> 4);
+    const int lx = (t & 7) | ((t >> 6) & 1) << 3, ly = ((t >> 3) & 7) | (t >> 7) << 3;
+    const int px = tx * 16 + lx, py = ty * 16 + ly;
     const bool inside = px < c.W && py < c.H;
     const uint32_t r0 = ranges[2 * tile], r1 = ranges[2 * tile + 1];
     float rd[3];
     pixel_dir((float)px + 0.5f, (float)py + 0.5f, c, rd);
     const float fx = (float)px + 0.5f, fy = (float)py + 0.5f;
+    const float X0 = (float)(tx * 16 + 8), Y0 = (float)(ty * 16 + 8);
+    const float ox = fx - X0, oy = fy - Y0;
 
     float T = 1.0f, C0 = 0.0f, C1 = 0.0f, C2 = 0.0f;
-    int cnt = 0, kc = 0, head = 0;
+    int cnt = 0, kc = 0;
     bool done = !inside;
+    // the k-buffer: depths in order, and in nibble k of ord the slot of entry k;
+    // it starts full of blanks that lie before every depth
+    float kd[KBUF];
+#pragma unroll
+    for (int k = 0; k < KBUF; k++) kd[k] = -__builtin_inff();
+    uint64_t ord = 0xfedcba9876543210ull;
+    // the entry blended last: its colour (in flight), alpha and transmittance
+    float w_r = 0.0f, w_g = 0.0f, w_b = 0.0f, w_a = 0.0f, w_T = 0.0f;
+    auto blend = [&](uint32_t sl, float a, float tt) {
+        C0 += w_r * w_a * w_T;
+        C1 += w_g * w_a * w_T;
+        C2 += w_b * w_a * w_T;
+        const float* col = rgb + (size_t)s_ki[sl][t] * 3;
+        w_r = col[0];
+        w_g = col[1];
+        w_b = col[2];
+        w_a = a;
+        w_T = T;
+        T = tt;
+        cnt++;
+    };
+
+    // threads 0 .. R3_BATCH-1 load one entry each, a round ahead
+    float4 n0, n1, n3;
+    float2 nc0, nc1, nc2;
+    float nm0, nm1, nm2, no, nd;
+    uint32_t nid = 0u;
+    auto load = [&](uint32_t j) {
+        if (t < R3_BATCH && j < r1) {
+            nid = values[j];
+            const float4* g4 = reinterpret_cast<const float4*>(g2s + (size_t)nid * 16);
+            n0 = g4[0];
+            n1 = g4[1];
+            n3 = g4[3];
+            const float2* c2 = reinterpret_cast<const float2*>(cinv + (size_t)nid * 6);
+            nc0 = c2[0];
+            nc1 = c2[1];
+            nc2 = c2[2];
+            nm0 = moff[(size_t)nid * 3];
+            nm1 = moff[(size_t)nid * 3 + 1];
+            nm2 = moff[(size_t)nid * 3 + 2];
+            no = op2d[nid];
+            nd = depths[nid];
+        }
+    };
+    load(r0 + t);
 
     for (uint32_t base = r0; base < r1; base += R3_BATCH) {
         // the workgroup stops once every pixel is finished
         if (__syncthreads_count(done ? 0 : 1) == 0) break;
-        const uint32_t j = base + t;
-        if (t < R3_BATCH && j < r1) {  // threads 0 .. R3_BATCH-1 stage one entry each
-            const uint32_t id = values[j];
-            const float4* g4 = reinterpret_cast<const float4*>(g2s + (size_t)id * 16);
-            Entry3& e = sm[t];
-            e.r0 = g4[0];
-            e.r1 = g4[1];
-            e.r3 = g4[3];
-            const float2* c2 = reinterpret_cast<const float2*>(cinv + (size_t)id * 6);
-            const float2 a = c2[0], b = c2[1], d = c2[2];
-            e.ci[0] = a.x; e.ci[1] = a.y; e.ci[2] = b.x; e.ci[3] = b.y; e.ci[4] = d.x; e.ci[5] = d.y;
-            e.mo[0] = moff[(size_t)id * 3];
-            e.mo[1] = moff[(size_t)id * 3 + 1];
-            e.mo[2] = moff[(size_t)id * 3 + 2];
-            const float o = op2d[id];
-            e.op = o;
-            e.depth = depths[id];
-            e.id = id;
-            e.cut = 1e-3f + __logf(255.0f * o);
+        if (t < R3_BATCH) {
+            Reach k = {1.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};  // behind the list's end: out of reach
+            if (base + t < r1) {
+                Entry3& e = sm[t];
+                e.r0 = n0;
+                e.r1 = n1;
+                e.r3 = n3;
+                e.ci[0] = nc0.x; e.ci[1] = nc0.y; e.ci[2] = nc1.x; e.ci[3] = nc1.y; e.ci[4] = nc2.x; e.ci[5] = nc2.y;
+                e.mo[0] = nm0;
+                e.mo[1] = nm1;
+                e.mo[2] = nm2;
+                e.op = no;
+                e.depth = nd;
+                e.id = nid;
+                k = reach_of(n0, n1, n3, no, X0, Y0);
+            }
+            s_q0[t] = make_float4(k.k00, k.k01, k.k02, k.k11);
+            s_q1[t] = make_float2(k.k12, k.k22);
         }
         __syncthreads();
-        const int m = (int)((r1 - base) < (uint32_t)R3_BATCH ? (r1 - base) : (uint32_t)R3_BATCH);
-        for (int q = 0; q < m && !done; q++) {
-            const Entry3& e = sm[q];
+        load(base + R3_BATCH + t);
+        uint64_t hits = 0u;  // bit q: entry q reaches this lane's pixel
+        if (!done) {
+            uint32_t half[2] = {0u, 0u};
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll 8
+                for (int q = 32 * h + 31; q >= 32 * h; q--) {
+#pragma clang fp contract(fast)
+                    const float4 a = s_q0[q];
+                    const float2 b = s_q1[q];
+                    const float v = ox * (ox * a.w + (oy * b.x + a.y)) + (oy * (oy * b.y + a.z) + a.x);
+                    half[h] = __builtin_amdgcn_alignbit(half[h], __float_as_uint(v), 31);  // its sign shifted in
+                }
+            hits = (uint64_t)half[1] << 32 | half[0];
+        }
+        while (hits) {
+            const Entry3& e = sm[__builtin_ctzll(hits)];
+            hits &= hits - 1u;
             const float plx[4] = {e.r0.x - e.r3.x * fx, e.r0.y - e.r3.y * fx, e.r0.z - e.r3.z * fx,
                                   e.r0.w - e.r3.w * fx};
             const float ply[4] = {e.r1.x - e.r3.x * fy, e.r1.y - e.r3.y * fy, e.r1.z - e.r3.z * fy,
                                   e.r1.w - e.r3.w * fy};
-            {
-                // Far below the 1/255 cut the exact evaluation can be skipped:
-                // |m|^2 rcp(dd) is within 1e-6 (relative) of the exact squared
-                // distance, so 0.5 md (1 - 1e-5) > 1e-3 + ln(255 o) gives
-                // o e^power < e^-0.001 / 255 for the exact power, which the
-                // exact path also skips (NaN and inf fall through or agree).
-                const float dx = plx[1] * ply[2] - plx[2] * ply[1];
-                const float dy = plx[2] * ply[0] - plx[0] * ply[2];
-                const float dz = plx[0] * ply[1] - plx[1] * ply[0];
+            // parallel planes: no distance (the division below would make a NaN)
+            const float dx = plx[1] * ply[2] - plx[2] * ply[1];
+            const float dy = plx[2] * ply[0] - plx[0] * ply[2];
+            const float dz = plx[0] * ply[1] - plx[1] * ply[0];
+            if (dx * dx + dy * dy + dz * dz == 0.0f) {
                 const float mx = plx[3] * ply[0] - plx[0] * ply[3];
                 const float my = plx[3] * ply[1] - plx[1] * ply[3];
                 const float mz = plx[3] * ply[2] - plx[2] * ply[3];
-                const float mm = mx * mx + my * my + mz * mz;  // must not overflow where the exact path does not
-                const float md = mm * __builtin_amdgcn_rcpf(dx * dx + dy * dy + dz * dz);
-                if (mm < 3.0e38f && 0.5f * md * (1.0f - 1e-5f) > e.cut) continue;
+                const float mm = mx * mx + my * my + mz * mz;
+                if (mm > 0.0f && mm < 3.0e38f) continue;
             }
             const float power = -0.5f * ray_contrib(plx, ply, nullptr);
             if (power > 0.0f) continue;
-            const float alpha = smin(0.99f, e.op * exp_ref_tab(power, s_e2));
+            const float alpha = smin(0.99f, e.op * exp_ref_nonpos(power, s_e2));
             if (alpha < kAlpha) continue;
             float pd = e.depth;
             if (c.have_ivp) {
                 const float ptd = depth_along(e.ci, e.mo, rd);
                 if (ptd > 0.0f) pd = ptd;
             }
+            // the front entry leaves: a blank until KBUF entries came
+            const uint32_t slot = (uint32_t)ord & 15u;
             if (kc >= KBUF) {
-                // blend the front entry (the buffer is full)
-                const float a = s_ka[head][t];
+                const float a = s_ka[slot][t];
                 const float tt = T * (1.0f - a);
                 if (tt < 0.0001f) {
                     done = true;
-                    continue;
+                    break;
                 }
-                const uint32_t gid = s_ki[head][t];
-                C0 += rgb[gid * 3] * a * T;
-                C1 += rgb[gid * 3 + 1] * a * T;
-                C2 += rgb[gid * 3 + 2] * a * T;
-                T = tt;
-                cnt++;
-                head = (head + 1) & (KBUF - 1);
-                kc = KBUF - 1;
+                blend(slot, a, tt);
+            } else {
+                kc++;
             }
-            // insertion after the last entry not deeper than pd
-            int at = kc;
-            while (at > 0) {
-                const int sl = (head + at - 1) & (KBUF - 1);
-                const float dprev = s_kd[sl][t];
-                if (!(dprev > pd)) break;
-                const int dst = (head + at) & (KBUF - 1);
-                s_kd[dst][t] = dprev;
-                s_ka[dst][t] = s_ka[sl][t];
-                s_ki[dst][t] = s_ki[sl][t];
-                at--;
+            // The new one goes behind the last entry not deeper than pd, so place k
+            // takes what was at k + 1 (the front left), or pd, or keeps its own.
+            // deeper: entry k and all behind it are deeper than pd.  Most insertions
+            // move an entry or two, so a group that no lane's pd passes only shifts.
+            int at = KBUF - 1;
+            float up = 0.0f;
+            bool deeper = true;
+#pragma unroll
+            for (int k0 = KBUF - R3_GROUP; k0 >= 0; k0 -= R3_GROUP) {
+                if (__any(deeper)) {
+#pragma unroll
+                    for (int k = k0 + R3_GROUP - 1; k >= k0; k--) {
+                        const float own = kd[k];
+                        const bool moves = deeper && k > 0 && own > pd;
+                        kd[k] = deeper ? (moves ? own : pd) : up;
+                        at -= moves ? 1 : 0;
+                        up = own;
+                        deeper = moves;
+                    }
+                } else {
+#pragma unroll
+                    for (int k = k0 + R3_GROUP - 1; k >= k0; k--) {
+                        const float own = kd[k];
+                        kd[k] = up;
+                        up = own;
+                    }
+                }
             }
-            const int dst = (head + at) & (KBUF - 1);
-            s_kd[dst][t] = pd;
-            s_ka[dst][t] = alpha;
-            s_ki[dst][t] = e.id;
-            kc++;
+            s_ka[slot][t] = alpha;
+            s_ki[slot][t] = e.id;
+            ord >>= 4;
+            const uint64_t low = ((uint64_t)1 << (4 * at)) - 1;
+            ord = (ord & low) | ((uint64_t)slot << (4 * at)) | ((ord & ~low) << 4);
         }
         __syncthreads();
     }
     if (!inside) return;
     // flush, front to back
     if (!done) {
-        for (int k = 0; k < kc; k++) {
-            const int sl = (head + k) & (KBUF - 1);
+        for (int k = KBUF - kc; k < KBUF; k++) {
+            const uint32_t sl = (uint32_t)(ord >> (4 * k)) & 15u;
             const float a = s_ka[sl][t];
             const float tt = T * (1.0f - a);
             if (tt < 0.0001f) break;
-            const uint32_t gid = s_ki[sl][t];
-            C0 += rgb[gid * 3] * a * T;
-            C1 += rgb[gid * 3 + 1] * a * T;
-            C2 += rgb[gid * 3 + 2] * a * T;
-            T = tt;
-            cnt++;
+            blend(sl, a, tt);
         }
     }
+    C0 += w_r * w_a * w_T;
+    C1 += w_g * w_a * w_T;
+    C2 += w_b * w_a * w_T;
     const int pix = py * c.W + px;
     if (T_final) T_final[pix] = T;
     if (n_contrib) n_contrib[pix] = cnt;

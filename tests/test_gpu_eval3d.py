@@ -195,3 +195,49 @@ def test_eval3d_fast_binning_errors(hip):
     pre_w, pre3d_w = hip.preprocess_3d(p, wide, cfg, raw=True)
     with pytest.raises(GsError, match="255"):
         hip.bin_tiles_3d(pre_w, pre3d_w, wide, capacity=1 << 20)
+
+
+@pytest.mark.parametrize("order", ["depth", "reversed", "shuffled"])
+@pytest.mark.parametrize("n,w,h,logscale,op", [
+    (1, 17, 9, (-2.0, 0.1), (2.0, 0.5)),       # one entry, ragged image
+    (63, 33, 31, (-1.0, 0.8), (0.0, 2.0)),     # one short of a staged round
+    (64, 16, 16, (-1.0, 0.8), (0.0, 2.0)),
+    (65, 48, 16, (-6.0, 0.3), (3.0, 1.0)),     # far smaller than a pixel
+    (300, 40, 24, (1.0, 1.5), (-5.5, 0.5)),    # larger than the view, opacities around 1/255
+    (700, 64, 40, (-2.5, 2.5), (-1.0, 3.0)),   # needles and sheets: every scale beside every other
+])
+def test_eval3d_raster_takes_any_list(hip, o3, n, w, h, logscale, op, order):
+    """Lists as no binning writes them: every tile holds every visible
+    Gaussian, whatever it reaches, in order of depth and against it, so that
+    the k-buffer inserts at each of its places; one entry has no finite plane
+    and some depths are infinite or NaN."""
+    _say("eval3d any list", n, w, h, order)
+    scene = gaussians_normal(n, 41 + n, 0, sigma=0.9, logscale=logscale, op=op)
+    cam = make_camera((0.2, -0.1, -3.0), w, h, 60.0)
+    cfg = RenderCfg(bg_color=(0.1, 0.2, 0.3), training=False, sh_degree=0)
+    pre, pre3d = hip.preprocess_3d(hip.upload_scene(scene), cam, cfg, raw=True)
+    hip.sync()
+    vis = np.flatnonzero(_np(pre["radii"]) > 0) if n > 1 else np.zeros(1, np.int64)
+    if n > 64:
+        pre["depths"][int(vis[3])] = float("inf")
+        pre["depths"][int(vis[7])] = float("nan")
+        pre3d["mean_offset"][int(vis[7])] = -pre3d["mean_offset"][int(vis[7])]  # no depth along the ray: its own
+        pre3d["g2s"].view(n, 16)[int(vis[11]), 0] = float("nan")
+    got = dict(means2D=_np(pre["means2D"]), depths=_np(pre["depths"]), op2d=_np(pre["op2d"]), rgb=_np(pre["rgb"]),
+               radii=_np(pre["radii"]), tiles=_np(pre["tiles"]), g2s=_np(pre3d["g2s"]),
+               cov3D_inv=_np(pre3d["cov3D_inv"]), mean_offset=_np(pre3d["mean_offset"]))
+    lst = vis[np.argsort(got["depths"][vis], kind="stable")]
+    if order == "reversed":
+        lst = lst[::-1]
+    elif order == "shuffled":
+        lst = np.random.default_rng(n).permutation(lst)
+    tiles = ((w + 15) // 16) * ((h + 15) // 16)
+    values = np.ascontiguousarray(np.tile(lst, tiles).astype(np.int32))
+    ranges = (np.arange(tiles)[:, None] * len(lst) + np.array([0, len(lst)])).astype(np.int32)
+    img, T, nc = hip.raster_fwd_3d(pre, pre3d, torch.from_numpy(values).to(hip.dev),
+                                   torch.from_numpy(ranges.reshape(-1).copy()).to(hip.dev), cam, tuple(cfg.bg_color))
+    hip.sync()
+    rimg, rT, rnc = o3.rasterize(got, values.view(np.uint32), ranges.view(np.uint32), cam, cfg.bg_color)
+    np.testing.assert_array_equal(_np(nc), rnc)
+    assert np.abs(_np(img) - rimg).max() <= IMAGE_TOL
+    assert np.abs(_np(T) - rT).max() <= IMAGE_TOL
