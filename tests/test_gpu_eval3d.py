@@ -241,3 +241,29 @@ def test_eval3d_raster_takes_any_list(hip, o3, n, w, h, logscale, op, order):
     np.testing.assert_array_equal(_np(nc), rnc)
     assert np.abs(_np(img) - rimg).max() <= IMAGE_TOL
     assert np.abs(_np(T) - rT).max() <= IMAGE_TOL
+
+
+@pytest.mark.parametrize("n,equal", [(1, False), (63, False), (511, False), (513, False), (8191, False), (8192, False),
+                                     (8193, False), (12000, False), (16384, False), (16385, False), (3000, True),
+                                     (9000, True)])
+def test_eval3d_tile_list_lengths(hip, o3, n, equal):
+    """One tile that every Gaussian touches, at the lengths where the list's
+    sort changes its workgroup, its rounds or its way; equal: one key only."""
+    _say("eval3d list length", n, equal)
+    scene = gaussians_normal(n, 7 + n, 0, sigma=0.02, logscale=(-1.0, 0.2), op=(2.0, 0.5))
+    if equal:
+        for a in (scene.pos, scene.log_scale, scene.rot, scene.opacity_logit):
+            a[:] = a[:1]
+    cam = make_camera((0.0, 0.0, -3.0), 16, 16, 60.0)
+    cfg = RenderCfg(training=False, sh_degree=0)
+    pre, pre3d = hip.preprocess_3d(hip.upload_scene(scene), cam, cfg, raw=True)
+    fv, fk, fr, K = hip.bin_tiles_3d(pre, pre3d, cam)
+    hip.sync()
+    assert K == n
+    got = dict(means2D=_np(pre["means2D"]), depths=_np(pre["depths"]), radii=_np(pre["radii"]),
+               tiles=_np(pre["tiles"]), cov3D_inv=_np(pre3d["cov3D_inv"]),
+               mean_offset=_np(pre3d["mean_offset"]))
+    sk, sv, sr = o3.sort(*o3.duplicate(got, n, cam), 1)
+    np.testing.assert_array_equal(_np(fv).view(np.uint32), sv)
+    np.testing.assert_array_equal(_np(fk).view(np.uint64), sk)
+    np.testing.assert_array_equal(_np(fr).view(np.uint32).reshape(-1, 2), sr)
