@@ -58,6 +58,11 @@ struct gs_batch {
     int persistent_groups = 0;
     uint32_t capacity = 0;
     bool direct = true;            // direct-placement binning (else the word sort)
+    // The depth sort's records: self-contained words index << (32 + view_bits) |
+    // view << 32 | depth where the index fits, else keys beside an index array.
+    // A pass moves 16 instead of 24 bytes per Gaussian and view (the passes of 16
+    // views of 1M Gaussians 813 -> 624 us, of 8 views of 6M 1799 -> 1428 us).
+    bool depth_words() const { return direct && (uint64_t)N <= 1ull << (32 - view_bits); }
     gsb::BinArgs bin{};            // direct placement: layout, views and workspace
     int num_cus = 0;
 
@@ -193,8 +198,14 @@ static int batch_setup_binning(gs_batch* b) {
         // a first guess (2 to 6 records per Gaussian and view are usual); batch_measure grows it
         B_TRY(batch_size_records(b, 4 * (size_t)V * b->N + 65536));
     }
-    a.sidx = b->didx_s.u();
-    a.sidx_stride = 1;
+    if (b->depth_words()) {
+        a.sidx = reinterpret_cast<const uint32_t*>(b->dkeys_s.p) + 1;
+        a.sidx_stride = 2;
+        a.sidx_shift = b->view_bits;
+    } else {
+        a.sidx = b->didx_s.u();
+        a.sidx_stride = 1;
+    }
     a.rect_idx = b->rect_idx.u();
     a.overflow = b->overflow();
     return GS_OK;
@@ -258,7 +269,8 @@ extern "C" int gs_batch_create(gs_trainer* tr, int n_views, const gs_camera* cam
         (st = b->counters.ensure(256)) || (st = b->means2D.ensure(VN * 8)) || (st = b->depths.ensure(VN * 4)) ||
         (st = b->conics.ensure(VN * 12)) || (st = b->op2d.ensure(VN * 4)) || (st = b->rgb.ensure(VN * 12)) ||
         (st = b->radii.ensure(VN * 4)) || (st = b->tiles.ensure(VN * 4)) || (st = b->dkeys.ensure(VN * 8)) ||
-        (st = b->didx.ensure(VN * 4)) || (st = b->dkeys_s.ensure(VN * 8)) || (st = b->didx_s.ensure(VN * 4)) ||
+        (st = b->dkeys_s.ensure(VN * 8)) ||
+        (!b->depth_words() && ((st = b->didx.ensure(VN * 4)) || (st = b->didx_s.ensure(VN * 4)))) ||
         (b->direct && (st = b->rect_idx.ensure(VN * 4))) ||
         (st = b->scan_partial.ensure(((VN + SCAN_BLOCK - 1) / SCAN_BLOCK + 1) * 8)) ||
         (st = b->dsort_ws.ensure(radix_workspace_bytes((uint32_t)VN, b->radix_bits))) ||
@@ -326,11 +338,14 @@ static int enqueue_binning(gs_batch* b, hipStream_t s, bool place = true) {
     gs_preprocessed pre = b->pre();
     const int deg = std::min(b->cfg.sh_degree, t->sh_degree);
     B_HIP(launch_preprocess_fwd_multi(g, static_cast<const gsd::CamArgs*>(b->cams_dev.p), b->V, pre,
-                                      static_cast<uint64_t*>(b->dkeys.p), b->didx.u(), deg, s,
+                                      static_cast<uint64_t*>(b->dkeys.p), b->depth_words() ? nullptr : b->didx.u(),
+                                      32 + b->view_bits, deg, s,
                                       b->direct ? b->rect_idx.u() : nullptr),
           "multi-view preprocess");
-    B_HIP(launch_radix_sort_bits(static_cast<const uint64_t*>(b->dkeys.p), b->didx.u(),
-                                 static_cast<uint64_t*>(b->dkeys_s.p), b->didx_s.u(), VN, 0, 32 + b->view_bits,
+    const bool words = b->depth_words();
+    B_HIP(launch_radix_sort_bits(static_cast<const uint64_t*>(b->dkeys.p), words ? nullptr : b->didx.u(),
+                                 static_cast<uint64_t*>(b->dkeys_s.p), words ? nullptr : b->didx_s.u(), VN, 0,
+                                 32 + b->view_bits,
                                  b->radix_bits, b->dsort_ws.p, s, nullptr),
           "depth sort");
     if (b->direct) {

@@ -479,7 +479,8 @@ struct BinArgs {
     int CH, C1;             // Gaussians per chunk, chunks per view (bin_layout)
     int GC, C2;             // chunks per group, groups per view (bin_layout)
     const uint32_t* sidx;   // [V*N]: each view's Gaussian indices in order, sidx_stride apart (null: index order)
-    int sidx_stride;        // 1: an index array; 2: the high words of sorted index << 32 | key words
+    int sidx_stride;        // 1: an index array; 2: the high words of sorted index << (32 + sidx_shift) | key words
+    int sidx_shift;         // key bits below the index in those high words (0 for an index array)
     const float2* means2D;  // view-major [V][N]
     const int* radii;       // [V][N]
     const uint32_t* rect_idx;  // optional [V][N]: packed rectangles by Gaussian index (else from means2D, radii)

@@ -124,7 +124,7 @@ hipError_t launch_zero(void* ptr, size_t bytes, hipStream_t s);
 
 // multi-view
 hipError_t launch_preprocess_fwd_multi(const gs_gaussians& G, const gsd::CamArgs* cams_dev, int V,
-                                       const gs_preprocessed& out, uint64_t* dkeys, uint32_t* didx, int deg,
+                                       const gs_preprocessed& out, uint64_t* dkeys, uint32_t* didx, int index_shift, int deg,
                                        hipStream_t s, uint32_t* rects = nullptr);
 hipError_t launch_preprocess_bwd_multi(const gs_gaussians& G, const gsd::CamArgs* cams_dev,
                                        const gsd::CamArgs* cam_val, int V, const int* radii, const gs_raster_grads& rg,

@@ -115,7 +115,7 @@ __device__ __forceinline__ int4 view_info(const BinArgs& a, int v) { return a.vi
 // (x0 | x1 << 8 | y0 << 16 | y1 << 24; 0 when culled).
 __device__ __forceinline__ uint2 rect_record(const BinArgs& a, int v, const int4& vi, uint32_t r) {
     const size_t seg = (size_t)v * a.N;
-    const uint32_t id = a.sidx ? a.sidx[(seg + r) * (size_t)a.sidx_stride] : r;
+    const uint32_t id = a.sidx ? a.sidx[(seg + r) * (size_t)a.sidx_stride] >> a.sidx_shift : r;
     if (a.rect_idx) return make_uint2(a.rect_idx[seg + id], id);  // packed beforehand, in index order
     const int rad = a.radii[seg + id];
     uint2 rec = make_uint2(0u, id);

@@ -143,14 +143,15 @@ __global__ __launch_bounds__(256) void preprocess_bwd_kernel(gs_gaussians G, Cam
 // ------------------------------------------------------------ multi-view ----
 // Forward over V views: parameters and SH read once, per-view outputs written
 // view-major ([v][N]), plus the depth-sort keys view << 32 | depth bits
-// (culled: view << 32 | 0xFFFFFFFF) and Gaussian indices; rects (optional,
+// (culled: view << 32 | 0xFFFFFFFF) and Gaussian indices, or, where didx is null,
+// the index in the key's bits from index_shift on; rects (optional,
 // views of at most 255 x 255 tiles): each Gaussian's packed tile rectangle
 // x0 | x1 << 8 | y0 << 16 | y1 << 24 (0 when culled), for the binning.
 template <int MAXC, int DEG>
 __global__ __launch_bounds__(256) void preprocess_fwd_multi_kernel(gs_gaussians G, const CamArgs* __restrict__ cams,
                                                                    int V, gs_preprocessed out,
                                                                    uint64_t* __restrict__ dkeys,
-                                                                   uint32_t* __restrict__ didx,
+                                                                   uint32_t* __restrict__ didx, int index_shift,
                                                                    uint32_t* __restrict__ rects) {
     constexpr int NB = (DEG + 1) * (DEG + 1);
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -185,8 +186,13 @@ __global__ __launch_bounds__(256) void preprocess_fwd_multi_kernel(gs_gaussians 
         out.rgb[o * 3] = rgb[0]; out.rgb[o * 3 + 1] = rgb[1]; out.rgb[o * 3 + 2] = rgb[2];
         out.radii[o] = radius;
         out.tiles_touched[o] = tiles;
-        dkeys[o] = ((uint64_t)v << 32) | (vis ? (uint64_t)__float_as_uint(depth) : 0xFFFFFFFFull);
-        didx[o] = (uint32_t)i;
+        const uint64_t key = ((uint64_t)v << 32) | (vis ? (uint64_t)__float_as_uint(depth) : 0xFFFFFFFFull);
+        if (didx) {
+            dkeys[o] = key;
+            didx[o] = (uint32_t)i;
+        } else {
+            dkeys[o] = ((uint64_t)i << index_shift) | key;
+        }
         if (rects) {
             uint32_t rec = 0u;
             if (radius > 0) {
@@ -485,13 +491,13 @@ hipError_t launch_preprocess_bwd(const gs_gaussians& G, const CamArgs& c, const 
 }
 
 hipError_t launch_preprocess_fwd_multi(const gs_gaussians& G, const CamArgs* cams_dev, int V,
-                                       const gs_preprocessed& out, uint64_t* dkeys, uint32_t* didx, int deg,
+                                       const gs_preprocessed& out, uint64_t* dkeys, uint32_t* didx, int index_shift, int deg,
                                        hipStream_t s, uint32_t* rects) {
     if (G.count <= 0) return hipSuccess;
     dim3 grid((G.count + 255) / 256), block(256);
     GS_DISPATCH_SH(G.max_coeffs, deg,
                    (preprocess_fwd_multi_kernel<MC, DG>
-                    <<<grid, block, 0, s>>>(G, cams_dev, V, out, dkeys, didx, rects)));
+                    <<<grid, block, 0, s>>>(G, cams_dev, V, out, dkeys, didx, index_shift, rects)));
     return hipGetLastError();
 }
 

@@ -204,3 +204,32 @@ def test_batched_word_sort_path_with_views_wider_than_255_tiles(hip):
         _, losses = b.result()
         assert np.allclose(losses, single_losses, rtol=0, atol=1e-6), (losses, single_losses)
         del b
+
+
+@pytest.mark.parametrize("views,n,radix_bits", [(1, 300, 8), (2, 8192, 8), (3, 5462, 8), (5, 700, 4), (5, 700, 5),
+                                                (9, 700, 6), (16, 700, 7), (17, 3000, 8)])
+def test_batch_depth_words_at_every_width(hip, views, n, radix_bits):
+    """The joint depth sort's words (index above view above depth) with each
+    digit width and number of view bits, above and below one workgroup's
+    sort: every view's image is the single-view render's, ties included."""
+    from gs_hip import GsBatch, GsTrainer
+    print("[case] batch depth words", views, n, radix_bits, flush=True)
+    scene, _, _ = random_small_scene(n, 1, 60 + views)
+    scene.pos[n // 2:n // 2 * 2] = scene.pos[:n // 2]  # equal depths keep index order
+    rng = np.random.Generator(np.random.Philox(views))
+    cams = [make_camera(sphere_eye(rng, 4.0), 70, 50, 60.0) for _ in range(views)]
+    gts = [target_image(c.width, c.height, i) for i, c in enumerate(cams)]
+    cfg = RenderCfg(sh_degree=1, training=True)
+    hip.set_tuning(radix_bits=radix_bits)
+    try:
+        tr = GsTrainer(hip, scene)
+        b = GsBatch(tr, cams, cfg, gts)
+        K = b.render()
+        got = [im.cpu().numpy() for im in b.images()]
+        total = 0
+        for v, cam in enumerate(cams):
+            total += tr.render(cam, cfg)
+            assert_image_close(got[v], tr.buffer("image", (cam.height, cam.width, 3)).cpu().numpy(), f"view {v}")
+        assert K == total
+    finally:
+        hip.set_tuning(radix_bits=8)
