@@ -613,7 +613,7 @@ __device__ __forceinline__ Reach reach_of(const float4& r0, const float4& r1, co
 // consecutive words) holds each one's alpha and id.  An insertion is the same few
 // instructions in every lane, where moving the deeper entries up one by one
 // through LDS waited for as many dependent reads as the wave's busiest lane
-// needed, and a third workgroup's worth of LDS is free for a fourth workgroup.
+// needed; and the LDS that the depths took makes room for a fourth workgroup.
 //
 // What bounds it is the issue of vector instructions: a pixel blends 73 of the
 // 330 entries that its tile visits (1M Gaussians, 1080p), at some 230
