@@ -195,7 +195,7 @@ static int batch_setup_binning(gs_batch* b) {
             return gs_set_error(GS_ERR_INVALID, "binning table too large");
         B_TRY(b->bin_ws.ensure(bin_workspace_bytes(a)));
         bin_carve(a, b->bin_ws.p);
-        // a first guess (2 to 6 records per Gaussian and view are usual); batch_measure grows it
+        // a first guess (2 to 6 records per Gaussian and view are usual); batch_measure sizes it
         B_TRY(batch_size_records(b, 4 * (size_t)V * b->N + 65536));
     }
     if (b->depth_words()) {
@@ -490,8 +490,9 @@ static int enqueue_step(gs_batch* b, hipStream_t s) {
     return GS_OK;
 }
 
-// Sizes the pair buffers from a binning pass (eager, synchronous): first the
-// record buffer, whose overflow cuts the pair count short, then the pairs.
+// Sizes the pair buffers from a binning pass (eager, synchronous), with a quarter
+// of headroom each: first the record buffer, whose overflow cuts the pair count
+// short, then the pairs.
 // The overflow flag is cleared when a buffer grew.
 static int batch_measure(gs_batch* b, long long* pairs) {
     if (b->capacity == 0) B_TRY(batch_size_pairs(b, 1024));
@@ -501,11 +502,15 @@ static int batch_measure(gs_batch* b, long long* pairs) {
         B_HIP(hipMemcpyAsync(&K, b->total64(), 8, hipMemcpyDeviceToHost, b->stream), "hipMemcpyAsync");
         B_HIP(hipMemcpyAsync(&records, b->records(), 8, hipMemcpyDeviceToHost, b->stream), "hipMemcpyAsync");
         B_HIP(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
-        if (b->direct && records > batch_record_cap(b)) {
+        if (b->direct) {
+            // a quarter of headroom, as the pairs have: the first steps spread the Gaussians
             if (records > 0xFFFFFFFFull) return gs_set_error(GS_ERR_CAPACITY, "more than 2^32-1 bin records");
-            B_TRY(batch_size_records(b, records + records / 4 + 65536));
-            B_HIP(launch_zero(b->overflow(), 4, b->stream), "zero overflow");
-            continue;
+            const bool fit = records <= batch_record_cap(b);
+            B_TRY(batch_size_records(b, (size_t)(records + records / 4 + 65536)));
+            if (!fit) {
+                B_HIP(launch_zero(b->overflow(), 4, b->stream), "zero overflow");
+                continue;
+            }
         }
         if (K > 0xFFFFFFFFull) return gs_set_error(GS_ERR_CAPACITY, "more than 2^32-1 pairs");
         *pairs = (long long)K;

@@ -132,3 +132,47 @@ def test_counted_binning_is_dropped_by_other_work(oracle):
     values = torch.empty(max(K.value, 1), dtype=torch.int32, device=hip.dev)
     ranges = torch.empty(2 * 13 * 7, dtype=torch.int32, device=hip.dev)
     assert hip.lib.gs_bin_tiles_place(hip.ctx, values.data_ptr(), values.numel(), ranges.data_ptr()) == 1
+
+
+def _covering_scene(n, wide, corner=0.0):
+    """n Gaussians, the first `wide` of them over all of a 1920 x 1024 view (480
+    bins, 7680 tiles, each); the rest behind the camera, or (corner, a size in
+    pixels) on the corners where four bins meet, two by two tiles over them."""
+    cam = make_camera((0.0, 0.0, -3.0), 1920, 1024, 60.0)
+    scene, _, _ = random_small_scene(n, 1, 5, op=(-4.0, 0.3))
+    rng = np.random.default_rng(n)
+    scene.pos[:] = rng.normal(0.0, 0.01, scene.pos.shape)
+    scene.log_scale[:] = np.log(0.9)
+    if corner:
+        f = cam.width / (2.0 * cam.tan_fovx) / 3.0  # pixels per unit at the origin
+        scene.pos[wide:, 0] = rng.integers(-14, 15, n - wide) * 64 / f
+        scene.pos[wide:, 1] = rng.integers(-7, 8, n - wide) * 64 / f
+        scene.pos[wide:, 2] = 0.0
+        scene.log_scale[wide:] = np.log(corner / f)
+    else:
+        scene.pos[wide:, 2] = -5.0
+    return scene, cam
+
+
+def _batch(hip, scene, cam):
+    from gs_hip import GsBatch, GsTrainer
+    tr = GsTrainer(hip, scene)
+    return tr, GsBatch(tr, [cam], RenderCfg(sh_degree=1, training=True), [target_image(cam.width, cam.height, 6)])
+
+
+def test_batch_records_have_headroom():
+    """A batch whose first measurement just fits the first guess of the record
+    buffer (4 a Gaussian and 65536: 66104) takes steps on Gaussians that need a
+    little more, as its pair buffer does."""
+    from gs_hip import GsHip, train_cfg
+    print("[case] batch record headroom", flush=True)
+    hip = GsHip(0)
+    scene, cam = _covering_scene(142, 137)  # 65760 records
+    tr, b = _batch(hip, scene, cam)
+    assert b.render() == 137 * 7680
+    grown, _ = _covering_scene(142, 142)    # 68160 records
+    tr.set_params(grown)
+    for i in range(3):
+        b.step(train_cfg(lr=1e-6), i)
+    res, _ = b.result()
+    assert res.pairs == 142 * 7680
