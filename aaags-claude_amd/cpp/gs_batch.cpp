@@ -490,6 +490,21 @@ static int enqueue_step(gs_batch* b, hipStream_t s) {
     return GS_OK;
 }
 
+// The counters of `small`, read back (waits for the batch's stream).
+struct BatchCounts {
+    uint32_t pairs32, unused;
+    unsigned long long pairs;
+    uint32_t overflow, skipped;
+    unsigned long long records;
+};
+
+static int batch_counts(gs_batch* b, BatchCounts* n) {
+    static_assert(sizeof(BatchCounts) == 32, "the layout of gs_batch::small");
+    B_HIP(hipMemcpyAsync(n, b->small.p, sizeof(*n), hipMemcpyDeviceToHost, b->stream), "hipMemcpyAsync(counts)");
+    B_HIP(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
+    return GS_OK;
+}
+
 // Sizes the pair buffers from a binning pass (eager, synchronous), with a quarter
 // of headroom each: first the record buffer, whose overflow cuts the pair count
 // short, then the pairs.
@@ -498,10 +513,9 @@ static int batch_measure(gs_batch* b, long long* pairs) {
     if (b->capacity == 0) B_TRY(batch_size_pairs(b, 1024));
     for (int attempt = 0; attempt < 2; attempt++) {
         B_TRY(enqueue_binning(b, b->stream, false));
-        unsigned long long K = 0, records = 0;
-        B_HIP(hipMemcpyAsync(&K, b->total64(), 8, hipMemcpyDeviceToHost, b->stream), "hipMemcpyAsync");
-        B_HIP(hipMemcpyAsync(&records, b->records(), 8, hipMemcpyDeviceToHost, b->stream), "hipMemcpyAsync");
-        B_HIP(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
+        BatchCounts n;
+        B_TRY(batch_counts(b, &n));
+        const unsigned long long K = n.pairs, records = n.records;
         if (b->direct) {
             // a quarter of headroom, as the pairs have: the first steps spread the Gaussians
             if (records > 0xFFFFFFFFull) return gs_set_error(GS_ERR_CAPACITY, "more than 2^32-1 bin records");
@@ -623,7 +637,9 @@ extern "C" int gs_batch_step(gs_batch* b, const gs_train_cfg* tc, int iteration,
     return GS_OK;
 }
 
-// Forward only for all views (the batched render).
+// Forward only for all views (the batched render).  With `pairs` the counts are
+// read back: a render whose lists were cut short, or its pair count with the bin
+// records, is measured again and repeated with larger buffers.
 extern "C" int gs_batch_render(gs_batch* b, long long* pairs) {
     if (!b) return gs_set_error(GS_ERR_INVALID, "null batch");
     gs_ctx* c = b->tr->ctx;
@@ -634,14 +650,22 @@ extern "C" int gs_batch_render(gs_batch* b, long long* pairs) {
         B_TRY(batch_measure(b, &K));
     }
     B_TRY(enqueue_forward(b, b->stream));
+    if (pairs) {
+        BatchCounts n;
+        B_TRY(batch_counts(b, &n));
+        *pairs = (long long)n.pairs;
+        if (n.pairs > b->capacity || n.records > batch_record_cap(b)) {
+            B_TRY(batch_measure(b, pairs));
+            B_TRY(enqueue_forward(b, b->stream));
+            // the flag was this render's, unless it kept queued steps from being
+            // applied: then it stays for their result
+            const uint32_t flag = n.skipped ? 1u : 0u;
+            B_HIP(hipMemcpyAsync(b->overflow(), &flag, 4, hipMemcpyHostToDevice, b->stream), "hipMemcpyAsync");
+            B_HIP(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
+        }
+    }
     B_HIP(hipEventRecord(b->ev_out, b->stream), "hipEventRecord");
     B_HIP(hipStreamWaitEvent(c->stream, b->ev_out, 0), "hipStreamWaitEvent");
-    if (pairs) {
-        unsigned long long K = 0;
-        B_HIP(hipMemcpyAsync(&K, b->total64(), 8, hipMemcpyDeviceToHost, b->stream), "hipMemcpyAsync");
-        B_HIP(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
-        *pairs = (long long)K;
-    }
     return GS_OK;
 }
 

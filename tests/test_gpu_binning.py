@@ -176,3 +176,52 @@ def test_batch_records_have_headroom():
         b.step(train_cfg(lr=1e-6), i)
     res, _ = b.result()
     assert res.pairs == 142 * 7680
+
+
+@pytest.mark.parametrize("n,wide,grown_wide,corner,what", [(200_000, 1000, 1000, 1.0, "records only"),
+                                                           (300, 20, 290, 0.0, "records and pairs"),
+                                                           (300, 20, 30, 0.0, "neither")])
+def test_batch_render_repeats_a_cut_render(n, wide, grown_wide, corner, what):
+    """A render after the parameters changed, whose records or pairs outgrow the
+    buffers that an earlier one sized: its count and image are the single
+    view's, and the next step is applied."""
+    from gs_hip import GsHip, GsTrainer, train_cfg
+    print("[case] batch render outgrows", what, flush=True)
+    hip = GsHip(0)
+    scene, cam = _covering_scene(n, wide)
+    tr, b = _batch(hip, scene, cam)
+    b.render()
+    grown, _ = _covering_scene(n, grown_wide, corner)
+    tr.set_params(grown)
+    K = b.render()
+    single = GsTrainer(hip, grown)
+    assert K == single.render(cam, RenderCfg(sh_degree=1, training=True))
+    assert torch.equal(b.images()[0], single.buffer("image", (cam.height, cam.width, 3)))
+    before = tr.params()[0].copy()
+    b.step(train_cfg(lr=1e-3), 0)
+    res, _ = b.result()
+    assert res.pairs == K
+    assert not np.array_equal(tr.params()[0], before)
+
+
+def test_batch_render_leaves_suppressed_steps_to_their_result():
+    """Steps that outgrew the buffers stay unapplied and reported after a render
+    that repeats itself with larger ones."""
+    from gs_hip import GsError, GsHip, train_cfg
+    print("[case] batch render between overflowed steps and their result", flush=True)
+    hip = GsHip(0)
+    scene, cam = _covering_scene(300, 20)
+    tr, b = _batch(hip, scene, cam)
+    b.render()
+    grown, _ = _covering_scene(300, 290)
+    tr.set_params(grown)
+    before = tr.params()[0].copy()
+    b.step(train_cfg(lr=1e-3), 0)
+    b.step(train_cfg(lr=1e-3), 1)
+    assert b.render() == 290 * 7680
+    with pytest.raises(GsError, match="2 step.s. were not applied"):
+        b.result()
+    assert np.array_equal(tr.params()[0], before)
+    b.step(train_cfg(lr=1e-3), 0)
+    b.result()
+    assert not np.array_equal(tr.params()[0], before)
