@@ -585,7 +585,10 @@ static int batch_result(gs_batch* b, gs_step_result* out, int iteration) {
         const uint32_t old_cap = b->capacity;
         if (b->direct) {
             // records that did not fit cut the pair count short: count again, growing both buffers
+            // (of the parameters as the trainer's stream leaves them, like a step)
             long long pairs = 0;
+            B_HIP(hipEventRecord(b->ev_in, b->tr->ctx->stream), "hipEventRecord");
+            B_HIP(hipStreamWaitEvent(b->stream, b->ev_in, 0), "hipStreamWaitEvent");
             B_TRY(batch_measure(b, &pairs));
             K = (unsigned long long)pairs;
             if (out) out->pairs = pairs;

@@ -225,3 +225,36 @@ def test_batch_render_leaves_suppressed_steps_to_their_result():
     b.step(train_cfg(lr=1e-3), 0)
     b.result()
     assert not np.array_equal(tr.params()[0], before)
+
+
+class _Array:
+    def __init__(self, address, shape):
+        self.__cuda_array_interface__ = dict(shape=tuple(shape), typestr="<f4", data=(address, False), version=3)
+
+
+def test_batch_result_measures_after_the_trainers_stream():
+    """The result of an overflowed step sizes the buffers from the parameters as
+    the work already queued on the trainer's stream leaves them, here behind a
+    tenth of a second of matrix products: the redo then fits."""
+    from gs_hip import GsError, GsHip, train_cfg
+    print("[case] batch result behind queued parameter writes", flush=True)
+    hip = GsHip(0)
+    scene, cam = _covering_scene(300, 20)
+    tr, b = _batch(hip, scene, cam)
+    b.render()
+    tr.set_params(_covering_scene(300, 100)[0])
+    more = torch.tensor(_covering_scene(300, 290)[0].pos, device=hip.dev)
+    pos = torch.as_tensor(_Array(tr.lib.gs_trainer_buffer(tr.tr, b"param_pos"), (300, 3)), device=hip.dev)
+    a = torch.zeros((8192, 8192), dtype=torch.bfloat16, device=hip.dev)
+    out = torch.empty_like(a)
+    torch.mm(a, a, out=out)
+    torch.cuda.synchronize()
+    b.step(train_cfg(lr=1e-6), 0)
+    for _ in range(100):
+        torch.mm(a, a, out=out)
+    pos.copy_(more)
+    with pytest.raises(GsError, match="not applied"):
+        b.result()
+    b.step(train_cfg(lr=1e-6), 0)
+    res, _ = b.result()
+    assert res.pairs == 290 * 7680
