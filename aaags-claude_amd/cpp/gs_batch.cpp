@@ -561,13 +561,11 @@ static int batch_upload_hparams(gs_batch* b, const gs_train_cfg* tc, int iterati
 // Reads the losses / pair count / overflow flag of the last step (synchronous).
 static int batch_result(gs_batch* b, gs_step_result* out, int iteration) {
     std::vector<double> L(b->V);
-    unsigned long long K = 0;
-    uint32_t flags[2] = {0, 0};  // overflow, suppressed updates
+    BatchCounts n;
     B_HIP(hipMemcpyAsync(L.data(), b->losses.p, 8 * b->V, hipMemcpyDeviceToHost, b->stream), "hipMemcpyAsync");
-    B_HIP(hipMemcpyAsync(&K, b->total64(), 8, hipMemcpyDeviceToHost, b->stream), "hipMemcpyAsync");
-    B_HIP(hipMemcpyAsync(flags, b->overflow(), 8, hipMemcpyDeviceToHost, b->stream), "hipMemcpyAsync");
-    B_HIP(hipStreamSynchronize(b->stream), "hipStreamSynchronize");
-    const uint32_t ovf = flags[0], skipped = flags[1];
+    B_TRY(batch_counts(b, &n));
+    unsigned long long K = n.pairs;
+    const uint32_t skipped = n.skipped;
     double s = 0.0;
     for (double x : L) s += x;
     if (out) {
@@ -576,13 +574,13 @@ static int batch_result(gs_batch* b, gs_step_result* out, int iteration) {
         out->n_gaussians = b->N;
         out->pairs = (long long)K;
     }
-    if (ovf) {
+    if (n.overflow) {
         // some step since the last check dropped pairs: that step and every
         // later one left the parameters and Adam state untouched; their Adam
         // step numbers are handed back, and the buffers grow for the redo
         B_HIP(launch_zero(b->overflow(), 8, b->stream), "zero overflow");
         b->tr->adam_steps -= (int)skipped;
-        const uint32_t old_cap = b->capacity;
+        const uint32_t old_cap = b->capacity, old_records = b->direct ? batch_record_cap(b) : 0u;
         if (b->direct) {
             // records that did not fit cut the pair count short: count again, growing both buffers
             // (of the parameters as the trainer's stream leaves them, like a step)
@@ -596,6 +594,11 @@ static int batch_result(gs_batch* b, gs_step_result* out, int iteration) {
         unsigned long long cap = K + K / 4 + 65536;
         if (cap > 0xFFFFFFFFull) cap = 0xFFFFFFFFull;
         B_TRY(batch_size_pairs(b, (uint32_t)cap));
+        if (b->direct && n.records > old_records && K <= old_cap)
+            return gs_set_error(GS_ERR_CAPACITY,
+                                "a batched step had %llu bin records for a capacity of %u: %u step(s) were not applied; "
+                                "buffers regrown to %u, repeat them",
+                                n.records, old_records, skipped, batch_record_cap(b));
         return gs_set_error(GS_ERR_CAPACITY,
                             "a batched step had %llu pairs for a capacity of %u: %u step(s) were not applied; "
                             "buffers regrown to %u, repeat them",
