@@ -207,7 +207,7 @@ static int batch_setup_binning(gs_batch* b) {
         a.sidx_stride = 1;
     }
     a.rect_idx = b->rect_idx.u();
-    a.overflow = b->overflow();
+    a.overflow = a.record_overflow = b->overflow();
     return GS_OK;
 }
 

@@ -362,13 +362,13 @@ static int tr_pairs(gs_trainer* t, long long* K, bool* fits) {
     bool records_fit = true;  // if not, the lists and K are cut short: the redo counts again
     TR_TRY(gs_bin_fits(t->ctx, *t->ctx->bin, counts[1], &records_fit));
     *fits = *fits && records_fit;
-    if (!*fits) {
+    if ((size_t)*K > cap) {
         // the dropped pairs raised the context's overflow flag: clear it, grow
         void* sm = nullptr;
         TR_TRY(gs_small_get(t->ctx, &sm));
         e = launch_zero(static_cast<char*>(sm) + GS_SMALL_OVERFLOW, 4, t->ctx->stream);
         if (e != hipSuccess) return gs_hip_status(e, "zero kernel");
-        if ((size_t)*K > cap) TR_TRY(t->keys_sorted.ensure((size_t)(*K + *K / 8 + 1024) * 4));
+        TR_TRY(t->keys_sorted.ensure((size_t)(*K + *K / 8 + 1024) * 4));
     }
     return GS_OK;
 }

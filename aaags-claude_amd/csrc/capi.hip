@@ -554,7 +554,6 @@ int gs_bin_count(gs_ctx* c, gsb::BinArgs& a, void* guess, unsigned long long* pa
         if ((st = gs_bin_fits(c, a, got[1], &fits))) return st;
         if (attempt > 0) return gs_set_error(GS_ERR_CAPACITY, "binning: the record buffer did not grow");
         if ((st = coarse_get(c, (size_t)got[1], a))) return st;
-        GS_HIP(launch_zero(a.overflow, 4, c->stream), "zero kernel");  // raised by the records that did not fit
     }
     *pairs = got[0];
     return GS_OK;

@@ -499,7 +499,8 @@ struct BinArgs {
     uint32_t coarse_cap;    // records
     uint32_t* out;          // Gaussian index per pair; 16-byte aligned
     uint32_t capacity;
-    uint32_t* overflow;     // raised when records or pairs outgrow their buffer
+    uint32_t* overflow;     // raised when pairs outgrow their buffer
+    uint32_t* record_overflow;  // raised when records do; null where the host reads their count anyway
 };
 }  // namespace gsb
 

@@ -211,7 +211,7 @@ __global__ __launch_bounds__(1024) void coarse_scan_kernel(uint32_t* __restrict_
 }
 
 // One block: the bins' first records (NB + 1 entries), the record count, and
-// the overflow flag when the records outgrow their buffer.
+// the flag (may be null) when the records outgrow their buffer.
 __global__ __launch_bounds__(1024) void coarse_starts_kernel(const uint32_t* __restrict__ tot, uint32_t NB,
                                                              uint32_t cap, uint32_t* __restrict__ start,
                                                              unsigned long long* __restrict__ total,
@@ -229,7 +229,7 @@ __global__ __launch_bounds__(1024) void coarse_starts_kernel(const uint32_t* __r
     if (threadIdx.x == 0) {
         start[NB] = (uint32_t)min(carry, (unsigned long long)0xFFFFFFFFu);
         *total = carry;
-        if (carry > cap) *overflow = 1u;
+        if (overflow && carry > cap) *overflow = 1u;
     }
 }
 
@@ -531,7 +531,8 @@ static hipError_t bin_lists(const BinArgs& a, hipStream_t s, unsigned long long*
     if (!counted) {
         coarse_count_kernel<BT><<<chunks, 256, 0, s>>>(a);
         coarse_scan_kernel<<<(a.NB + 15) / 16, 1024, 0, s>>>(a.table1, a.C1, a.NB, a.tot);
-        coarse_starts_kernel<<<1, 1024, 0, s>>>(a.tot, a.NB, a.coarse_cap, a.start, records, a.overflow);
+        coarse_starts_kernel<<<1, 1024, 0, s>>>(a.tot, a.NB, a.coarse_cap, a.start, records,
+                                                a.record_overflow);
     }
     if (a.max_bins <= 256)
         coarse_place_kernel<BT, 256><<<chunks, 256, 0, s>>>(a);

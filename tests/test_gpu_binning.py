@@ -300,3 +300,30 @@ def test_batch_step_whose_records_alone_outgrow_their_buffer(graph):
         if k not in ("adam_m_rot", "adam_v_rot"):  # the scales are equal: no rotation gradient but rounding
             # float atomics in another order: 1e-3, as gradients between runs
             assert np.linalg.norm(x - want[k]) <= 1e-3 * np.linalg.norm(want[k]), k
+
+
+@pytest.mark.parametrize("who", ["bin_tiles", "trainer"])
+def test_growing_records_keep_the_overflow_flag(who):
+    """Pairs that gs_duplicate_keys dropped are still reported after a binning
+    whose bin records outgrew their buffer and were counted again."""
+    from gs_hip import GsHip, GsTrainer
+    print("[case] overflow flag kept", who, flush=True)
+    hip = GsHip(0)
+    small = {k: torch.tensor(v, device=hip.dev) for k, v in _pre(300, 200, 100, 30, 9).items()}
+    # 48000 records, then 87600 for a first guess of 80000; the trainer's pairs keep fitting
+    scene, cam = _covering_scene(10_000, 100)
+    grown, _ = _covering_scene(10_000, 100, 1.0)
+    cfg = RenderCfg(sh_degree=1, training=True)
+    if who == "trainer":
+        tr = GsTrainer(hip, scene)
+        tr.render(cam, cfg)
+        tr.set_params(grown)
+    offsets, K = hip.scan_tiles(small["tiles"])
+    hip.duplicate(small, offsets, K, 200, 100, capacity=K - 1)
+    if who == "trainer":
+        K = tr.render(cam, cfg)
+    else:
+        _, _, K = hip.bin_tiles(hip.preprocess(hip.upload_scene(grown), cam, cfg), cam.width, cam.height)
+    assert K == 100 * 7680 + 9900 * 4
+    assert hip.check_overflow()
+    assert not hip.check_overflow()
