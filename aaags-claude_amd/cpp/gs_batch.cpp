@@ -147,9 +147,9 @@ static int batch_size_pairs(gs_batch* b, uint32_t cap) {
     return GS_OK;
 }
 
-// Room for `records` bin records.
+// Room for `records` bin records, or for one per Gaussian and bin.
 static int batch_size_records(gs_batch* b, size_t records) {
-    records = std::min<size_t>(records, 0xFFFFFFFFu);
+    records = std::min(records, std::min<size_t>((size_t)b->N * b->bin.NB, 0xFFFFFFFFu));
     const size_t bytes = records * bin_record_bytes(b->bin);
     if (bytes <= b->coarse.bytes) return GS_OK;
     b->graph.release();

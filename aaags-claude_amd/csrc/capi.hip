@@ -500,13 +500,13 @@ extern "C" int gs_ctx_apply_tuning(gs_ctx* c, const gs_tuning* t) {
 }
 
 // First guess for the record buffer, in records per Gaussian (6 at 1M
-// Gaussians and 1080p).  That many lie behind the binning's tables in its
-// workspace, so most contexts allocate nothing more; a view that needs more
-// gets a buffer of its own, which then stays.
+// Gaussians and 1080p; at most one per bin).  That many lie behind the binning's
+// tables in its workspace, so most contexts allocate nothing more; a view that
+// needs more gets a buffer of its own, which then stays.
 constexpr size_t kRecordsPerGaussian = 8;
 
 size_t gs_bin_guess_bytes(const gsb::BinArgs& a) {
-    return (size_t)a.V * a.N * kRecordsPerGaussian * bin_record_bytes(a) + 256;
+    return (size_t)a.V * a.N * std::min<size_t>(kRecordsPerGaussian, (size_t)a.max_bins) * bin_record_bytes(a) + 256;
 }
 
 // Record buffer for the binning whose workspace ends with `guess`

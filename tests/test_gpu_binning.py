@@ -327,3 +327,26 @@ def test_growing_records_keep_the_overflow_flag(who):
     assert K == 100 * 7680 + 9900 * 4
     assert hip.check_overflow()
     assert not hip.check_overflow()
+
+
+def test_workspace_of_a_view_with_few_bins():
+    """A Gaussian has one record per bin at most: a view of one bin reserves an
+    eighth of the records that a view of eight or more does."""
+    from gs_hip import GsHip
+    print("[case] record workspace", flush=True)
+    n = 1_000_000
+
+    def used(width):
+        dev = {k: torch.tensor(v, device="cuda") for k, v in _pre(n, width, 64, 3, 1).items()}
+        hip = GsHip(0)
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        hip.bin_tiles(dev, width, 64)
+        torch.cuda.synchronize()
+        got = free - torch.cuda.mem_get_info()[0]
+        del hip, dev
+        torch.cuda.empty_cache()
+        return got
+
+    used(64)  # code objects and torch's own pools
+    assert used(512) - used(64) >= 7 * 8 * n
