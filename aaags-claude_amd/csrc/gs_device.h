@@ -476,7 +476,7 @@ struct BinArgs {
     int side;               // tiles per bin side, 4 or 8 (bin_side)
     uint32_t NB;            // bins over all views
     int max_bins;           // bins of the largest view
-    int CH, C1;             // Gaussians per chunk, chunks per view (bin_layout)
+    int S, CH, C1;          // first chunks, of 256 Gaussians; Gaussians per later chunk; chunks per view (bin_layout)
     int GC, C2;             // chunks per group, groups per view (bin_layout)
     const uint32_t* sidx;   // [V*N]: each view's Gaussian indices in order, sidx_stride apart (null: index order)
     int sidx_stride;        // 1: an index array; 2: the high words of sorted index << (32 + sidx_shift) | key words

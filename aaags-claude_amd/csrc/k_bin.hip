@@ -11,7 +11,7 @@
 // Two levels, because a Gaussian covers tens of tiles but few bins of 4 x 4
 // tiles (47 tiles, 6 bins on average at 1M Gaussians, 1080p):
 //
-//   level 1, bin lists: the depth order is cut into chunks of CH Gaussians.
+//   level 1, bin lists: the depth order is cut into chunks (bin_layout).
 //     coarse_count:  per (chunk, bin) the Gaussians whose rectangle meets the
 //                    bin, by a difference array over the bin grid in LDS (four
 //                    LDS atomics per Gaussian, whatever its size).
@@ -128,20 +128,33 @@ __device__ __forceinline__ uint2 rect_record(const BinArgs& a, int v, const int4
     return rec;
 }
 
+// Depth ranks [r0, r1) of chunk c: the first S chunks hold 256, the others CH.
+__device__ __forceinline__ void chunk_ranks(const BinArgs& a, int c, uint32_t& r0, uint32_t& r1) {
+    const int late = max(c - a.S, 0);
+    r0 = 256u * (uint32_t)(c - late) + (uint32_t)a.CH * (uint32_t)late;
+    r1 = min(r0 + (c < a.S ? 256u : (uint32_t)a.CH), (uint32_t)a.N);
+}
+
 // One block per (view, chunk): the depth-ordered rectangle records of the
 // chunk and its count in every bin of the view.
+//
+// Here and in coarse_place the chunks go round the XCDs one by one, not in a run
+// to each: the nearest chunks have the most records and the last ones, of culled
+// Gaussians, none, so with runs one XCD had most of the work (4M Gaussians, 1.7M
+// of them in view, 1080p: coarse_count 61 -> 41 us, coarse_place 133 -> 91; 1M,
+// all in view: 12.6 -> 12.7 and 54.6 -> 50.9).
 template <int BT>
 __global__ __launch_bounds__(256) void coarse_count_kernel(BinArgs a) {
     __shared__ int dif[2 * GS_BIN_MAX_BINS];  // (columns + 1) x (rows + 1)
-    const int q = gsd::xcd_remap(blockIdx.x, gridDim.x);
+    const int q = blockIdx.x;
     const int v = q / a.C1, c = q - v * a.C1;
     const int4 vi = view_info(a, v);
     const int nbx = (vi.x + BT - 1) / BT, nby = (vi.y + BT - 1) / BT, W1 = nbx + 1;
     const int tid = threadIdx.x;
     for (int i = tid; i < W1 * (nby + 1); i += 256) dif[i] = 0;
     __syncthreads();
-    const uint32_t r0 = (uint32_t)c * (uint32_t)a.CH;
-    const uint32_t r1 = min(r0 + (uint32_t)a.CH, (uint32_t)a.N);
+    uint32_t r0, r1;
+    chunk_ranks(a, c, r0, r1);
     for (uint32_t r = r0 + (uint32_t)tid; r < r1; r += 256u) {
         const uint2 rec = rect_record(a, v, vi, r);
         a.rects[(size_t)v * a.N + r] = rec;
@@ -246,7 +259,7 @@ __global__ __launch_bounds__(256) void coarse_place_kernel(BinArgs a) {
     __shared__ uint32_t s_cur[MAXB];      // per bin: the next record
     using Rec = typename Bins<BT>::Rec;
     Rec* const coarse = reinterpret_cast<Rec*>(a.coarse);
-    const int q = gsd::xcd_remap(blockIdx.x, gridDim.x);
+    const int q = blockIdx.x;
     const int v = q / a.C1, c = q - v * a.C1;
     const int4 vi = view_info(a, v);
     const int nbx = (vi.x + BT - 1) / BT, nby = (vi.y + BT - 1) / BT, nb = nbx * nby;
@@ -257,8 +270,8 @@ __global__ __launch_bounds__(256) void coarse_place_kernel(BinArgs a) {
 #pragma unroll
         for (int k = 0; k < 4; k++) s_m[k][b] = 0ull;
     }
-    const uint32_t r0 = (uint32_t)c * (uint32_t)a.CH;
-    const uint32_t r1 = min(r0 + (uint32_t)a.CH, (uint32_t)a.N);
+    uint32_t r0, r1;
+    chunk_ranks(a, c, r0, r1);
     const uint2* rects = a.rects + (size_t)v * a.N;
     uint2 nxt = r0 + (uint32_t)tid < r1 ? rects[r0 + tid] : make_uint2(0u, 0u);
     __syncthreads();
@@ -488,7 +501,12 @@ int bin_count_of_view(int side, int gx, int gy) { return ((gx + side - 1) / side
 
 // Chunks: 256 .. 4096 Gaussians, the largest that still gives 512 chunks (two
 // blocks per CU) so that small scenes spread over the chip and large ones keep
-// the (chunk, bin) table small.  Groups: enough level-2 blocks to fill the
+// the (chunk, bin) table small; 2048 at most while that table has 32 MB or less,
+// and the first 128 chunks, of the nearest Gaussians, 256: from inside a scene
+// those meet tens of bins each (43 on average in the first thousand, 4 over all)
+// and one block of 4096 of them outlasted all others (4M Gaussians, 1.7M in view,
+// 1080p: coarse_place 353 us; 154 with the near chunks cut, 91 with both).
+// Groups: enough level-2 blocks to fill the
 // chip several times (8192) and about one per 512 Gaussians beyond, so that
 // the bins where a scene is densest do not leave one long block at the end; in
 // views of few bins up to one per 128 Gaussians, since with 64 groups a bin the
@@ -498,9 +516,13 @@ int bin_count_of_view(int side, int gx, int gy) { return ((gx + side - 1) / side
 void bin_layout(BinArgs& a) {
     const size_t vn = (size_t)a.V * (size_t)a.N;
     int rounds = 1;
-    while (rounds < 16 && vn / (256u * 2u * (size_t)rounds) >= 512u) rounds *= 2;
+    while (rounds < 16 && vn / (256u * 2u * (size_t)rounds) >= 512u) {
+        if (rounds >= 8 && ((size_t)a.N / (256u * (size_t)rounds) + 1u) * a.NB * 4u <= (size_t)32 << 20) break;
+        rounds *= 2;
+    }
     a.CH = 256 * rounds;
-    a.C1 = (a.N + a.CH - 1) / a.CH;
+    a.S = rounds > 1 ? std::min(128, a.N / 2048) : 0;
+    a.C1 = a.S + (a.N - 256 * a.S + a.CH - 1) / a.CH;
     const size_t blocks = std::min(std::max<size_t>(8192u, vn / 512u), std::max<size_t>(vn / 128u, (size_t)64u * a.NB));
     const int want = (int)std::max<size_t>(blocks / a.NB, 1u);
     a.GC = (a.C1 + want - 1) / want;

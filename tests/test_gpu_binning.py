@@ -31,8 +31,9 @@ def _pre(n, width, height, max_radius, seed):
     (1, 16, 16, 30), (255, 64, 64, 40), (256, 65, 64, 40), (257, 80, 130, 100), (5000, 411, 307, 60),
     (2048, 200, 100, 20), (2049, 200, 100, 20), (16384, 300, 200, 10), (16385, 300, 200, 10),  # sort in one workgroup, or not
     (131_072, 500, 400, 8), (131_073, 500, 400, 8),  # digit counts scanned in the scatter, or in a launch
-    (140_000, 500, 400, 12),            # chunks of 512 Gaussians
+    (140_000, 500, 400, 12),            # 547 chunks of 256 Gaussians
     (140_000, 64, 64, 6), (140_001, 66, 20, 6),  # one bin and two: a group per chunk
+    (262_143, 500, 400, 6), (262_144, 500, 400, 6), (262_657, 64, 64, 4),  # 128 chunks of 256, then of 512
     (3000, 2048, 2048, 300),            # 1024 bins of 4 x 4 tiles
     (3000, 2064, 2048, 300),            # bins of 8 x 8 tiles
     (500, 4080, 4080, 900),             # the largest view: 255 x 255 tiles
