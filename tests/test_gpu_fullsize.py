@@ -69,32 +69,22 @@ def test_1m_16views_batched_render_equals_single_views(hip):
         assert torch.equal(imgs[v], single), f"view {v}"
 
 
-def test_fullsize_two_round_forward_equals_one_round(hip):
-    """1M Gaussians, 1920x1080: the trainer's two-round forward (64 groups of
-    1024 depth-ordered Gaussians first) and the one-round forward give the
-    same image, T_final, contributor counts and last contributors, bit for
-    bit."""
+def test_1m_1080p_trainer_render_equals_stage_chain(hip, scene_1m_1080p):
+    """1M Gaussians, 1920x1080: the trainer's forward (two-level binning; first
+    with the pair count read back, then without waiting for it) gives the image,
+    T_final, contributor counts, last contributors and pair count of the stage
+    chain (scan, duplicate-with-keys, 64-bit pair sort, raster), bit for bit."""
     from gs_hip import GsTrainer
-    from gs_scenes import RenderCfg, make_workload
-    print("[case] full-size two-round forward", flush=True)
-    scene, cams, _ = make_workload("1m_1080p")
-    cam = cams[0]
+    print("[case] 1m 1080p trainer render vs stage chain", flush=True)
+    scene, cam, _ = scene_1m_1080p
     cfg = RenderCfg(sh_degree=3, training=True)
-    out = []
-    try:
-        for sp in (0, 64):
-            hip.set_split(sp)
-            tr = GsTrainer(hip, scene)
-            tr.render(cam, cfg)
-            K = tr.render(cam, cfg)
-            torch.cuda.synchronize()
-            H, W = cam.height, cam.width
-            out.append((K, [tr.buffer("image", (H, W, 3)), tr.buffer("T_final", (H, W)),
-                            tr.buffer("n_contrib", (H, W), torch.int32),
-                            tr.buffer("last_contrib", (H, W), torch.int32)]))
-            del tr
-    finally:
-        hip.set_split(64)  # the context default
-    assert out[0][0] == out[1][0]
-    for a, b in zip(out[0][1], out[1][1]):
-        assert torch.equal(a, b)
+    f = hip.forward(hip.upload_scene(scene), cam, cfg)
+    tr = GsTrainer(hip, scene)
+    H, W = cam.height, cam.width
+    for _ in range(2):
+        assert tr.render(cam, cfg) == f["K"]
+        torch.cuda.synchronize()
+        assert torch.equal(tr.buffer("image", (H, W, 3)), f["img"])
+        assert torch.equal(tr.buffer("T_final", (H, W)), f["px"]["T_final"].view(H, W))
+        assert torch.equal(tr.buffer("n_contrib", (H, W), torch.int32), f["px"]["n_contrib"].view(H, W))
+        assert torch.equal(tr.buffer("last_contrib", (H, W), torch.int32), f["px"]["last_contrib"].view(H, W))

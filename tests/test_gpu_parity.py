@@ -145,12 +145,10 @@ def test_depth_ordered_binning_bitexact(hip, oracle, n, deg, seed, radix_bits):
 
 
 @pytest.mark.parametrize("n,deg,seed", SMALL_CASES[1:] + [(10000, 0, 0)])
-@pytest.mark.parametrize("group,tpl", [(256, 1), (256, 2), (1024, 4), (16384, 2)])
-def test_direct_binning_bitexact(hip, oracle, n, deg, seed, group, tpl):
+def test_direct_binning_bitexact(hip, oracle, n, deg, seed):
     """gs_bin_tiles: values and ranges equal to the reference's
-    duplicate-with-keys + stable 64-bit sort, bit for bit, with several
-    groups per view (256) and with one (16384), for every bin shape."""
-    _say("direct binning", n, deg, seed, group, tpl)
+    duplicate-with-keys + stable 64-bit sort, bit for bit."""
+    _say("direct binning", n, deg, seed)
     if n == 10000:
         scene, cams, _ = make_workload("10k_256")
         cam = cams[0]
@@ -164,11 +162,7 @@ def test_direct_binning_bitexact(hip, oracle, n, deg, seed, group, tpl):
     keys_ref, vals_ref = oracle.duplicate(ref, scene.n, cam.width, cam.height)
     ks_ref, vs_ref, rg_ref = oracle.sort_pairs(keys_ref, vals_ref, cam.num_tiles)
     pre = _to_dev(hip, {k: ref[k] for k in ["means2D", "depths", "conics", "op2d", "rgb", "radii", "tiles"]})
-    hip.set_binning(group, tpl)
-    try:
-        vals, ranges, K = hip.bin_tiles(pre, cam.width, cam.height)
-    finally:
-        hip.set_binning(4096, 1)  # the context defaults
+    vals, ranges, K = hip.bin_tiles(pre, cam.width, cam.height)
     assert K == len(keys_ref)
     assert np.array_equal(u32(vals), vs_ref)
     assert np.array_equal(u32(ranges), rg_ref)
@@ -176,10 +170,9 @@ def test_direct_binning_bitexact(hip, oracle, n, deg, seed, group, tpl):
 
 @pytest.mark.parametrize("width,height", [(2080, 2080), (2032, 2032)])
 def test_direct_binning_bitexact_large_view(hip, oracle, width, height):
-    """Both ways of counting (tile, group) pairs: 2032 x 2032 (127 x 127
-    tiles) is counted with the LDS difference array, 2080 x 2080 (130 x 130
-    tiles) is over its size and uses the per-bin walk.  Values and ranges
-    equal the reference's duplicate + stable sort."""
+    """Both bin sizes: 2032 x 2032 (127 x 127 tiles) has 1024 bins of 4 x 4
+    tiles, 2080 x 2080 (130 x 130 tiles) would have more and takes bins of 8 x 8.
+    Values and ranges equal the reference's duplicate + stable sort."""
     _say("direct binning large view", width, height)
     scene, cam, _ = random_small_scene(3000, 1, 23, width=width, height=height)
     cfg = RenderCfg(sh_degree=3, training=True)
@@ -189,11 +182,7 @@ def test_direct_binning_bitexact_large_view(hip, oracle, width, height):
     ks_ref, vs_ref, rg_ref = oracle.sort_pairs(keys_ref, vals_ref, cam.num_tiles)
     assert len(keys_ref) > 10000
     pre = _to_dev(hip, {k: ref[k] for k in ["means2D", "depths", "conics", "op2d", "rgb", "radii", "tiles"]})
-    hip.set_binning(256, 2)
-    try:
-        vals, ranges, K = hip.bin_tiles(pre, cam.width, cam.height)
-    finally:
-        hip.set_binning(4096, 1)
+    vals, ranges, K = hip.bin_tiles(pre, cam.width, cam.height)
     assert K == len(keys_ref)
     assert np.array_equal(u32(vals), vs_ref)
     assert np.array_equal(u32(ranges), rg_ref)

@@ -163,43 +163,32 @@ def _render_state(tr, cam):
             tr.buffer("last_contrib", (H, W), torch.int32).cpu().numpy()]
 
 
-@pytest.mark.parametrize("split", [1, 3, 20])
-def test_trainer_two_round_forward_equals_one_round(hip, oracle, split):
-    """The trainer's two-round forward (the nearest `split` depth groups placed
-    and rendered first, the rest placed only for bins with unfinished tiles)
-    gives the one-round forward's image and pixel state bit for bit, and the
-    step then matches the oracle.  A dense scene (most tiles finish in round
-    1) with small groups (256 Gaussians, 80 groups)."""
+def test_trainer_dense_scene_render_and_step(hip, oracle):
+    """A dense scene whose tiles mostly finish early in their lists: a render
+    whose pair count is read back and one that does not wait for it give the same
+    image and pixel state bit for bit, and a step of the second kind the
+    oracle's loss, image and gradients."""
     from gs_hip import GsTrainer, train_cfg
-    print("[case] two-round forward", split, flush=True)
+    print("[case] dense scene", flush=True)
     scene, cam, gt = random_small_scene(20000, 3, 41, width=160, height=128, logscale=(-2.0, 0.4), op=(0.6, 1.0))
     cfg = RenderCfg(sh_degree=3, training=True)
     gt_t = torch.tensor(gt, device=hip.dev)
-    hip.set_binning(256, 1)
-    try:
-        states = []
-        for sp in (0, split):
-            hip.set_split(sp)
-            tr = GsTrainer(hip, scene)
-            K = tr.render(cam, cfg)
-            K = tr.render(cam, cfg)  # the second render uses the asynchronous pair count
-            torch.cuda.synchronize()
-            states.append((K, _render_state(tr, cam)))
-        assert states[0][0] == states[1][0]
-        for a, b in zip(states[0][1], states[1][1]):
-            assert np.array_equal(a, b)
-        # an SGD step with the split (the second one: its pair count is
-        # asynchronous): the oracle's loss, image and gradients
-        hip.set_split(split)
-        tr2 = GsTrainer(hip, scene)
-        tr2.step(cam, cfg, gt_t, train_cfg(use_adam=False), 0)
+    states = []
+    tr = GsTrainer(hip, scene)
+    for _ in range(2):  # the first render reads the pair count back, the second does not wait for it
+        K = tr.render(cam, cfg)
         torch.cuda.synchronize()
-        p1 = tr2.params()
-        res = tr2.step(cam, cfg, gt_t, train_cfg(use_adam=False), 0)
-        torch.cuda.synchronize()
-    finally:
-        hip.set_binning(4096, 1)
-        hip.set_split(64)  # the context default
+        states.append((K, _render_state(tr, cam)))
+    assert states[0][0] == states[1][0]
+    for a, b in zip(states[0][1], states[1][1]):
+        assert np.array_equal(a, b)
+    # the second of two SGD steps does not wait for its pair count either
+    tr2 = GsTrainer(hip, scene)
+    tr2.step(cam, cfg, gt_t, train_cfg(use_adam=False), 0)
+    torch.cuda.synchronize()
+    p1 = tr2.params()
+    res = tr2.step(cam, cfg, gt_t, train_cfg(use_adam=False), 0)
+    torch.cuda.synchronize()
     n = scene.n
     from gs_scenes import RawScene
     mid = RawScene(p1[0], p1[1], p1[2], p1[3].reshape(scene.sh.shape), p1[4], scene.sh_degree)
