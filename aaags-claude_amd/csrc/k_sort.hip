@@ -30,8 +30,8 @@ constexpr int SCAN_BLOCK = SCAN_THREADS * SCAN_ITEMS;  // 4096
 constexpr int RS_THREADS = 256;
 constexpr int RS_WAVES = RS_THREADS / 64;
 // Keys per block = 256 threads x ROUNDS: 4096 for large sorts (long output
-// runs per digit), 1024 below 4M keys so that a sort of ~1M keys still spreads
-// over ~1000 blocks instead of ~250.
+// runs per digit), 2048 below 4M keys so that a sort of ~1M keys still spreads
+// over ~500 blocks instead of ~250.
 constexpr uint32_t RS_SMALL_LIMIT = 1u << 22;
 // Sorts of at most this many blocks scan the digit counts inside the scatter
 // (rs_downsweep_kernel, DIRECT): 58.7 -> 53.2 us at 50k keys and four passes,
@@ -1132,22 +1132,15 @@ static hipError_t sort_pass_d(const uint64_t* ki, const uint32_t* vi, uint64_t* 
     return hipGetLastError();
 }
 
-template <int BITS, int ROUNDS>
-static hipError_t sort_pass_r(const uint64_t* ki, const uint32_t* vi, uint64_t* ko, uint32_t* vo, uint32_t n,
-                              const uint32_t* n_dev, int shift, uint32_t* hist, uint32_t* goff,
-                              uint32_t* dtot, hipStream_t s) {
-    if (radix_blocks(n) <= RS_DIRECT_BLOCKS)
-        return sort_pass_d<BITS, ROUNDS, true>(ki, vi, ko, vo, n, n_dev, shift, hist, goff, dtot, s);
-    return sort_pass_d<BITS, ROUNDS, false>(ki, vi, ko, vo, n, n_dev, shift, hist, goff, dtot, s);
-}
-
 template <int BITS>
 static hipError_t sort_pass(const uint64_t* ki, const uint32_t* vi, uint64_t* ko, uint32_t* vo, uint32_t n,
                             const uint32_t* n_dev, int shift, uint32_t* hist, uint32_t* goff, uint32_t* dtot,
                             hipStream_t s) {
-    if (radix_rounds(n) == 16) return sort_pass_r<BITS, 16>(ki, vi, ko, vo, n, n_dev, shift, hist, goff, dtot, s);
-    if (radix_rounds(n) == 8) return sort_pass_r<BITS, 8>(ki, vi, ko, vo, n, n_dev, shift, hist, goff, dtot, s);
-    return sort_pass_r<BITS, 4>(ki, vi, ko, vo, n, n_dev, shift, hist, goff, dtot, s);
+    if (radix_rounds(n) == 16)  // 4M keys and more: 1024 blocks at least
+        return sort_pass_d<BITS, 16, false>(ki, vi, ko, vo, n, n_dev, shift, hist, goff, dtot, s);
+    if (radix_blocks(n) <= RS_DIRECT_BLOCKS)
+        return sort_pass_d<BITS, 8, true>(ki, vi, ko, vo, n, n_dev, shift, hist, goff, dtot, s);
+    return sort_pass_d<BITS, 8, false>(ki, vi, ko, vo, n, n_dev, shift, hist, goff, dtot, s);
 }
 
 static hipError_t single_sort(const uint64_t* ki, uint64_t* ko, uint32_t n, const uint32_t* n_dev, const int* shifts,
