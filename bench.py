@@ -206,7 +206,7 @@ def bench_batched(hip, cfg, args):
     # batched, graph-captured step
     tr = GsTrainer(hip, scene)
     b = GsBatch(tr, cams, cfg, gts, persistent=True, fused_adam=True, use_graph=True)
-    tuning = None if args.no_autotune else b.autotune(reps=2)
+    tuning = None if args.no_autotune else knobs(b.autotune(reps=2))
     for i in range(2):
         b.step(tc, i, sync=True)
     steps = max(2, args.steps // 2)
@@ -362,6 +362,11 @@ def raster_work(hip, tr, scene, cam, cfg):
     return w
 
 
+def knobs(tuning):
+    """A tuning as it is reported: without the knobs that are stored and change nothing."""
+    return tuning and {k: v for k, v in tuning.items() if k not in ("bin_group", "bin_tiles_per_lane", "split_groups")}
+
+
 def cpu_model():
     """The host CPU's model name (/proc/cpuinfo), or the platform string."""
     try:
@@ -454,12 +459,12 @@ def traffic_probe(args):
     tr.set_options(fused_adam=True)
     # the autotuner runs every rasterizer instance (LDS batch depth), so the
     # counters cover the instance the timed benchmark picks
-    tuning = tr.autotune(cam, cfg, gt, reps=5)
+    tuning = knobs(tr.autotune(cam, cfg, gt, reps=5))
     if args.probe_tuning:
         # fixed knobs for the measured steps: counter passes slow every
         # dispatch down, so the autotuner may pick differently from pass to pass
         hip.apply_tuning({k: int(v) for k, v in (kv.split("=") for kv in args.probe_tuning.split(","))})
-        tuning = hip.tuning()
+        tuning = knobs(hip.tuning())
     tc = train_cfg(lr=1e-3)
     for i in range(2):
         r = tr.step(cam, cfg, gt, tc, i)
@@ -490,9 +495,8 @@ def main():
     ap.add_argument("--traffic-probe", action="store_true",
                     help="only run each stage kernel and a 1 GiB device copy (for rocprofv3 --pmc runs)")
     ap.add_argument("--probe-tuning", default="",
-                    help="with --traffic-probe: knobs for the measured steps, as key=value,key=value (every knob of "
-                         "gs_tuning: radix_bits, raster_batch, raster_bwd_batch, bin_group, bin_tiles_per_lane, "
-                         "persistent_per_cu, split_groups)")
+                    help="with --traffic-probe: knobs for the measured steps, as key=value,key=value "
+                         "(radix_bits, raster_batch, raster_bwd_batch, persistent_per_cu)")
     ap.add_argument("--large-workload", default="6m_8x1080p")
     ap.add_argument("--no-eval3d", action="store_true", help="skip the eval_3D (k-buffer) forward leg")
     ap.add_argument("--eval3d-only", action="store_true",
@@ -543,7 +547,7 @@ def main():
     tuning = None
     if not args.no_autotune:
         t0 = time.perf_counter()
-        tuning = tr.autotune(cam, cfg, gt, reps=5)
+        tuning = knobs(tr.autotune(cam, cfg, gt, reps=5))
         log(f"autotune ({time.perf_counter() - t0:.1f}s): {tuning}")
     for i in range(args.warmup):
         r = tr.step(cam, cfg, gt, tc, i)
@@ -632,7 +636,8 @@ def main():
         if insts:
             # secondary: VALU issue occupancy (instructions executed, from the committed
             # rocprofv3 SQ_INSTS_VALU summary, per second against 4 cycles per
-            # wave64 instruction); a measure of how busy the SIMDs are, not of work done
+            # wave64 instruction); a measure of how busy the SIMDs are, not of work
+            # done.  It can pass 1: not every counted instruction takes 4 cycles
             ach = insts / sec / 1e9
             roofline["valu_issue"] = {"achieved": round(ach, 1), "peak": round(VALU_WAVE_INSTS_PER_S / 1e9, 1),
                                       "unit": "G VALU wave-instructions/s",
