@@ -142,11 +142,13 @@ __device__ __forceinline__ void chunk_ranks(const BinArgs& a, int c, uint32_t& r
 // to each: the nearest chunks have the most records and the last ones, of culled
 // Gaussians, none, so with runs one XCD had most of the work (4M Gaussians, 1.7M
 // of them in view, 1080p: coarse_count 61 -> 41 us, coarse_place 133 -> 91; 1M,
-// all in view: 12.6 -> 12.7 and 54.6 -> 50.9).
+// all in view: 12.6 -> 12.7 and 54.6 -> 50.9).  From eight views on a run is a
+// whole view or more, and this kernel keeps the runs: the rectangles it gathers
+// from are then in one L2 (16 views of 1M: 156 us against 235).
 template <int BT>
 __global__ __launch_bounds__(256) void coarse_count_kernel(BinArgs a) {
     __shared__ int dif[2 * GS_BIN_MAX_BINS];  // (columns + 1) x (rows + 1)
-    const int q = blockIdx.x;
+    const int q = a.V >= 8 ? gsd::xcd_remap(blockIdx.x, gridDim.x) : (int)blockIdx.x;
     const int v = q / a.C1, c = q - v * a.C1;
     const int4 vi = view_info(a, v);
     const int nbx = (vi.x + BT - 1) / BT, nby = (vi.y + BT - 1) / BT, W1 = nbx + 1;
