@@ -716,10 +716,10 @@ extern "C" int gs_batch_info(gs_batch* b, int* total_tiles, long long* total_pix
 // ------------------------------------------------------------ autotuning ----
 // Coordinate descent over the batch's knobs, each timed on its own stage with
 // HIP events on the batch's stream (median of `reps` runs after one untimed
-// run): binning bin shape and group size (binning pass), persistent groups per
-// CU (forward + backward raster; 0 = one group per tile) and the LDS batch
-// depths of the two rasterizers.  Parameters and optimizer state are not
-// touched: only binning, forward, loss and backward raster run.
+// run): persistent groups per CU (forward + backward raster; 0 = one group per
+// tile) and the LDS batch depths of the two rasterizers; the binning pass is
+// timed once.  Parameters and optimizer state are not touched: only binning,
+// forward, loss and backward raster run.
 namespace {
 
 struct BatchTimer {

@@ -42,7 +42,7 @@
 // One level (a wave per group of Gaussians and 8 x 8-tile bin, one visit per
 // Gaussian and bin, 15 of 64 lanes live) took 377 us for those 47M pairs, and
 // 275 us where a first raster round let it skip part of them; these kernels
-// take 59 (coarse_place), 26 (tile_count) and 65 us (tile_place), 2.9 TB/s of
+// take 53 (coarse_place), 26 (tile_count) and 67 us (tile_place), 2.8 TB/s of
 // pairs.  At 10k Gaussians and 256 x 256 pixels placement went from 165 to
 // 5 us, at 1M and 4K from 1004 to 261 us, at 16 views of 1M (371M pairs) from
 // 2740 to 869 us.
@@ -490,10 +490,10 @@ __global__ __launch_bounds__(256) void bin_ranges_kernel(const uint32_t* __restr
 
 using namespace gsb;
 
-// Views of up to 1024 bins of 4 x 4 tiles (2048 x 2048 pixels, say) use those, larger views bins of 8 x 8: the bin masks of a block then
-// always fit a few workgroups per CU, and the larger rectangles of a larger
-// view meet as many bins as before (at 4K, 1M Gaussians: 6.9 records per
-// Gaussian instead of 18).
+// Views of up to 1024 bins of 4 x 4 tiles (2048 x 2048 pixels, say) use those,
+// larger views bins of 8 x 8: the bin masks of a block then always fit a few
+// workgroups per CU, and the larger rectangles of a larger view meet as many bins
+// as before (at 4K, 1M Gaussians: 6.9 records per Gaussian instead of 18).
 int bin_side(int max_gx, int max_gy) {
     const int b4 = ((max_gx + 3) / 4) * ((max_gy + 3) / 4);
     return b4 <= GS_BIN_MAX_BINS ? 4 : 8;

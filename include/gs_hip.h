@@ -470,13 +470,16 @@ int gs_batch_set_options(gs_batch* b, int persistent, int fused_adam, int use_gr
 int gs_batch_set_targets(gs_batch* b, const float* const* targets, int from_host);
 /* One batched step with Adam.  out == NULL: no host synchronisation (results
  * and the capacity check are read by a later gs_batch_result / step with out).
- * A step whose pairs exceed the pre-sized buffers updates nothing (its
- * backward and Adam kernels skip on the device's overflow word, and its Adam
+ * A step whose pairs or bin records exceed the pre-sized buffers updates
+ * nothing (its backward and Adam kernels skip on the device's overflow word, and its Adam
  * step count is rolled back); the next check returns GS_ERR_CAPACITY, regrows
  * the buffers, and the caller repeats the steps that were not applied. */
 int gs_batch_step(gs_batch* b, const gs_train_cfg* tc, int iteration, gs_step_result* out);
 int gs_batch_result(gs_batch* b, gs_step_result* out, double* view_losses);
-/* Forward only for all views into the batch's concatenated image buffer. */
+/* Forward only for all views into the batch's concatenated image buffer.  With
+ * pairs != NULL the pair count is read back (a host wait), and a render that
+ * outgrew the buffers is repeated with larger ones; without, such a render's
+ * lists are cut short and the next gs_batch_result reports it. */
 int gs_batch_render(gs_batch* b, long long* pairs);
 void* gs_batch_buffer(gs_batch* b, const char* which);
 int gs_batch_info(gs_batch* b, int* total_tiles, long long* total_pixels, long long* capacity);
